@@ -86,16 +86,17 @@ enum { PH_CHECK = 0, PH_STAGE1 = 1 };
 // The reciprocal of the rational tanh's denominator d >= 1, as 1 - 1/d needs it: 1/d
 // rounded to nearest for 1 <= d < 2^25, from the hardware reciprocal estimate (within
 // 1 ulp) and one Newton-Raphson step r + r(1 - d r) evaluated with fused multiply-adds
-// (Markstein's correction); 0 for d >= 2^25 (and +inf), where 1/d <= 2^-25 and 1 - 1/d
-// rounds to 1 either way. A NaN stays a NaN. Five instructions instead of the general
+// (Markstein's correction); 2^-25 for d >= 2^25 (and +inf), where 1/d <= 2^-25 and 1 - 1/d
+// rounds to 1 either way (one v_minimum3_f32, which keeps a NaN, where a comparison and a
+// selection were two instructions). Four instructions instead of the general
 // IEEE division's scale/fixup sequence; ccnn_selftest_tanh checks the reciprocal against
 // IEEE division on every float in [1, 2^25) and the tanh on every float.
 __device__ __forceinline__ float recip_ge1(float d)
 {
-    const float r = __builtin_amdgcn_rcpf(d);
-    const float e = __builtin_fmaf(-d, r, 1.f);
-    const float q = __builtin_fmaf(e, r, r);
-    return d >= 33554432.f ? 0.f : q;
+    const float x = __builtin_elementwise_minimum(d, 33554432.f);
+    const float r = __builtin_amdgcn_rcpf(x);
+    const float e = __builtin_fmaf(-x, r, 1.f);
+    return __builtin_fmaf(e, r, r);
 }
 
 template <bool IEEE_DIV = false>
@@ -1093,6 +1094,35 @@ __global__ void __launch_bounds__(256) k_cmp_emit(const float* __restrict__ resp
     }
 }
 
+// A lane's value from another lane of its row of 16 (DPP: one VALU instruction, where a
+// shuffle goes through the LDS unit).
+enum { DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140 };
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+// the largest value of a row of 16 lanes, in all of them
+__device__ __forceinline__ float row_max(float v)
+{
+    v = fmaxf(v, dpp<DPP_XOR1>(v));
+    v = fmaxf(v, dpp<DPP_XOR2>(v));
+    v = fmaxf(v, dpp<DPP_HALF_MIRROR>(v));
+    return fmaxf(v, dpp<DPP_MIRROR>(v));
+}
+// inclusive prefix sums over the 64 lanes of a wave: four shifted adds inside each row of
+// 16 lanes, then the row totals broadcast to the rows after them
+__device__ __forceinline__ int wave_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);      // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);      // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);      // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // row_bcast:15, rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);      // row_bcast:31, rows 2 and 3
+    return v;
+}
+
 // ---------------------------------------------------------------------------------
 // Stages 2/3: one workgroup evaluates one candidate's whole check
 // (CPUCheckDetect without the order-dependent drop logic, which the host replays).
@@ -1113,18 +1143,16 @@ constexpr int WL = Stage2::SIZE > Stage3::SIZE ? Stage2::SIZE : Stage3::SIZE;
 
 // LDS of one (candidate, crop variant). Regions are reused as their contents die:
 //   in  the network input; after L1 the L2 maps; after the L2 sums the L3 maps
-//       followed by the output
 //   s1  the crop's histogram and LUT while the crop is prepared; then the L1 sums;
 //       after L2 the L2 sums; after L3 the hidden layer
 //   w   the weights of the running network (stage 2 or 3)
 struct ChkSmem {
     alignas(16) float in[chk::IH * chk::IW];
     alignas(16) float s1[6 * chk::P1N];
-    float w[chk::WL];
-    float w3[Stage3::SIZE];  // k_check: the stage-3 weights beside the stage-2 ones in w
+    alignas(16) float w[chk::WL];
+    alignas(16) float w3[Stage3::SIZE];  // k_check: the stage-3 weights beside the stage-2 ones in w
     __device__ float* p2() { return in; }
     __device__ float* a3() { return in; }
-    __device__ float* out() { return in + 24 * chk::RN; }
     __device__ float* s2() { return s1; }
     __device__ float* h() { return s1; }
     __device__ int* hist() { return reinterpret_cast<int*>(s1); }
@@ -1363,9 +1391,20 @@ __device__ __forceinline__ void check_l1l2_mfma(const float* __restrict__ in, Ch
     __syncthreads();
 }
 
+// One network on one input. What bounds it: with one or two workgroups on a CU a wave issues
+// an instruction every ~5 clocks, so a phase lasts as long as its busiest wave and every
+// LDS wait on the way; with four it is the VALU's issue. So the positions that do not fill
+// whole waves are spread over all waves (one wave had 289 instructions more than the
+// others), the L3 and output operands are read ahead of their chains in 16-byte loads (78
+// waits became 28: 2.9 -> 1.2 us an item), two hidden units share an item (1.5 -> 0.9 us) and
+// the outcome is taken from the first wave's registers. k_check on 1920x1080 frames of
+// ~570 items: 37.2 -> 35.2 us alone, 18.6 -> 16.6 us a frame in a batch of 64; on 640x480
+// 28.4 -> 24.0 us.
+// Returns {responses above thr, bits of the largest response (at least -10)} in the first
+// wave's threads; out (optional) gets the RN responses.
 template <class N, int RP = RP_EXACT>
-__device__ __forceinline__ void check_forward(const float* __restrict__ in, ChkSmem& s,
-                                              const float* Wl, const int tid,
+__device__ __forceinline__ int2 check_forward(const float* __restrict__ in, ChkSmem& s,
+                                              const float* Wl, const int tid, float thr, float* out = nullptr,
                                               const float* __restrict__ mw = nullptr, int* s_red = nullptr)
 {
     using namespace chk;
@@ -1376,11 +1415,15 @@ __device__ __forceinline__ void check_forward(const float* __restrict__ in, ChkS
     if constexpr (RP != RP_EXACT) {
         check_l1l2_mfma<N, RP>(in, s, Wl, tid, mw, s_red);
     } else {
-    // L1 + sums: the first FULL positions one per lane (whole waves), the REM others by
-    // one wave with a lane per 2x2-pool quad. Index arithmetic is unsigned throughout.
-    constexpr unsigned FULL = P1N / 64 * 64, REM = P1N - FULL;
-    static_assert(REM == 0 || REM * 4 == 64, "the remainder fills one wave, four lanes a position");
-    for (unsigned p = ut; p < FULL; p += CHECK_THREADS) {
+    // L1 + sums: each wave takes a quarter of the positions, whole waves of them with one
+    // position per lane; the PREM that are left are computed by four lanes a position (one
+    // per 2x2-pool quad), a third of the maps each, so that no wave waits for another's
+    // remainder. Index arithmetic is unsigned throughout.
+    constexpr unsigned WAVES = CHECK_THREADS / 64, PW = P1N / WAVES, PREM = PW % 64;
+    static_assert(P1N % WAVES == 0 && PREM == 4 && N::M1 == 6, "remainder: 4 positions x 4 quads x 3 map pairs");
+    const unsigned wave = ut >> 6, lane = ut & 63u;
+    for (unsigned w0 = lane; w0 < PW - PREM; w0 += 64) {
+        const unsigned p = wave * PW + w0;
         const unsigned py = p / P1W, px = p - py * P1W;
         float win[5][5];
 #pragma unroll
@@ -1407,32 +1450,35 @@ __device__ __forceinline__ void check_forward(const float* __restrict__ in, ChkS
         for (int i = 1; i < N::M1 - 1; ++i) s.s1[i * P1N + p] = pm[i - 1] + pm[i] + pm[i + 1];
         s.s1[(N::M1 - 1) * P1N + p] = pm[N::M1 - 2] + pm[N::M1 - 1];
     }
-    if (REM > 0 && ut < REM * 4) {
-        const unsigned p = FULL + (ut >> 2), q = ut & 3u;
+    {
+        // lane = 16 * map pair + 4 * position + quad (the last 16 lanes repeat pair 2)
+        const unsigned g = min(lane >> 4, 2u), q = lane & 3u;
+        const unsigned p = wave * PW + PW - PREM + ((lane >> 2) & 3u);
         const unsigned py = p / P1W, px = p - py * P1W;
         const unsigned dx = q & 1u, dy = q >> 1;
-        float win[4][4];
+        float win[16];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
+        for (int j = 0; j < 16; ++j) win[j] = in[(2 * py + dy + (j >> 2)) * IW + 2 * px + dx + (j & 3)];
+        float pm[2];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) win[r][c] = in[(2 * py + dy + r) * IW + 2 * px + dx + c];
-        float pm[N::M1];
-#pragma unroll
-        for (int m = 0; m < N::M1; ++m) {
+        for (int h = 0; h < 2; ++h) {
+            const unsigned m = 2 * g + h;
             const float* k = Wl + N::oK1 + m * 16;
-            float acc = win[0][0] * k[0];
+            float acc = win[0] * k[0];
 #pragma unroll
-            for (int j = 1; j < 16; ++j) acc = acc + win[j >> 2][j & 3] * k[j];
+            for (int j = 1; j < 16; ++j) acc = acc + win[j] * k[j];
             const float a = lrelu_bn(acc, Wl + N::oB1, m, N::M1);
             // fmaxf(fmaxf(a0, a1), fmaxf(a2, a3)) across the position's four lanes
-            const float m01 = fmaxf(a, __shfl_xor(a, 1, 64));
-            pm[m] = fmaxf(m01, __shfl_xor(m01, 2, 64));
+            const float m01 = fmaxf(a, dpp<DPP_XOR1>(a));
+            pm[h] = fmaxf(m01, dpp<DPP_XOR2>(m01));
         }
-        if (q == 0) {
-            s.s1[p] = pm[0] + pm[1];
-#pragma unroll
-            for (int i = 1; i < N::M1 - 1; ++i) s.s1[i * P1N + p] = pm[i - 1] + pm[i] + pm[i + 1];
-            s.s1[(N::M1 - 1) * P1N + p] = pm[N::M1 - 2] + pm[N::M1 - 1];
+        // the neighbouring pairs' maps 2g - 1 and 2g + 2
+        const float before = __shfl(pm[1], (int)lane - 16, 64), after = __shfl(pm[0], (int)lane + 16, 64);
+        if (q == 0 && lane < 48) {
+            const float b = g > 0 ? before + pm[0] : pm[0];     // pm[2g - 1] + pm[2g]
+            const float c = pm[0] + pm[1];
+            s.s1[2 * g * P1N + p] = b + pm[1];
+            s.s1[(2 * g + 1) * P1N + p] = g < 2 ? c + after : c;
         }
     }
     __syncthreads();
@@ -1478,21 +1524,38 @@ __device__ __forceinline__ void check_forward(const float* __restrict__ in, ChkS
     }
     __syncthreads();
     PHASE(PH_CHECK, PB + 2);
-    // L3: conv_8x7 single chain (cnnpp_cplusplus.cpp:292-321) + lrelu_bn
-    for (unsigned it = ut; it < N::M2 * RN; it += CHECK_THREADS) {
-        const unsigned i = it / RN, p = it - i * RN;
+    // L3: conv_8x7 single chain (cnnpp_cplusplus.cpp:292-321) + lrelu_bn. The window and
+    // the weights (16-byte loads) are all read ahead of the chains
+    static_assert(N::M2 * RN <= CHECK_THREADS && N::K3W * N::K3H % 4 == 0 && N::oK3 % 4 == 0, "one L3 item per thread");
+    if (ut < N::M2 * RN) {
+        constexpr int K3N = N::K3W * N::K3H;
+        const unsigned i = ut / RN, p = ut - i * RN;
         const unsigned y = p / RW, x = p - y * RW;
         const float* src = s2 + i * P2N + y * P2W + x;
+        const float* k = Wl + N::oK3 + 2 * i * K3N;
+        float v[K3N], acc[2];
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int m = 2 * i + half;
-            const float* k = Wl + N::oK3 + m * N::K3W * N::K3H;
-            float acc = src[0] * k[0];
+        for (int j = 0; j < K3N; ++j) v[j] = src[(j / N::K3W) * P2W + (j % N::K3W)];
+        float4 w[2][2];              // four taps of both maps in use, the next four on their way
+        const auto fetch = [&](int g) {
 #pragma unroll
-            for (int j = 1; j < N::K3W * N::K3H; ++j)
-                acc = acc + src[(j / N::K3W) * P2W + (j % N::K3W)] * k[j];
-            s.a3()[m * RN + p] = lrelu_bn(acc, Wl + N::oB3, m, N::M3);
+            for (int h = 0; h < 2; ++h) w[g & 1][h] = *reinterpret_cast<const float4*>(k + h * K3N + 4 * g);
+        };
+        fetch(0);
+#pragma unroll
+        for (int g = 0; g < K3N / 4; ++g) {
+            if (g + 1 < K3N / 4) fetch(g + 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float4 t = w[g & 1][h];
+                acc[h] = g == 0 ? v[0] * t.x : acc[h] + v[4 * g] * t.x;
+                acc[h] = acc[h] + v[4 * g + 1] * t.y;
+                acc[h] = acc[h] + v[4 * g + 2] * t.z;
+                acc[h] = acc[h] + v[4 * g + 3] * t.w;
+            }
         }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) s.a3()[(2 * i + h) * RN + p] = lrelu_bn(acc[h], Wl + N::oB3, 2 * i + h, N::M3);
     }
     __syncthreads();
     PHASE(PH_CHECK, PB + 3);
@@ -1501,41 +1564,79 @@ __device__ __forceinline__ void check_forward(const float* __restrict__ in, ChkS
     // layer's serial sum over u reads its terms with 16-byte loads issued together
     constexpr int HLP = (N::HL + 3) / 4 * 4;
     static_assert(HLP * RN <= 6 * P1N, "the output-layer terms fit the s1 region");
-    for (unsigned it = ut; it < N::HL * RN; it += CHECK_THREADS) {
-        const unsigned u = it / RN, p = it - u * RN;
+    // two units of a group per item, so that they share the inputs and their chains overlap
+    static_assert(N::HLS % 2 == 0 && N::HLN % 4 == 0 && N::oHW % 4 == 0, "pairs of hidden units");
+    const auto hidden = [&](unsigned it) {
+        const unsigned u = it / RN * 2, p = it % RN;
         const unsigned gi = u / N::HLS, tt = u - gi * N::HLS;
-        float c = Wl[N::oHB + u];
+        float x[N::HLN], o[2];
 #pragma unroll
-        for (int j = 0; j < N::HLN; ++j) c = c + s.a3()[(gi + j) * RN + p] * Wl[N::oHW + u * N::HLN + j];
-        c = c * Wl[N::oHT + gi];
-        c = rtanh(c);
-        c = (c + 1.f) * 0.5f;
-        const float hv = Wl[N::oHBW + tt] * c + Wl[N::oHBB + tt];
-        s.h()[p * HLP + u] = hv * Wl[N::oOW + tt * N::HLG + gi];
-    }
+        for (int j = 0; j < N::HLN; ++j) x[j] = s.a3()[(gi + j) * RN + p];
+        const float tw = Wl[N::oHT + gi];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float c = Wl[N::oHB + u + h];
+#pragma unroll
+            for (int j = 0; j < N::HLN; ++j) c = c + x[j] * Wl[N::oHW + (u + h) * N::HLN + j];
+            c = c * tw;
+            c = rtanh(c);
+            c = (c + 1.f) * 0.5f;
+            const float hv = Wl[N::oHBW + tt + h] * c + Wl[N::oHBB + tt + h];
+            o[h] = hv * Wl[N::oOW + (tt + h) * N::HLG + gi];
+        }
+        *reinterpret_cast<float2*>(s.h() + p * HLP + u) = make_float2(o[0], o[1]);
+    };
+    constexpr unsigned HI = N::HL / 2 * RN;
+#pragma unroll
+    for (unsigned r = 0; r < HI / CHECK_THREADS; ++r) hidden(ut + r * CHECK_THREADS);
+    if (ut < HI % CHECK_THREADS) hidden(ut + HI / CHECK_THREADS * CHECK_THREADS);
     __syncthreads();
     PHASE(PH_CHECK, PB + 4);
     // output layer: the products in unit order, summed serially (the first term alone,
-    // then term + sum: IEEE addition commutes, so the order of the sum is what counts)
-    if (tid < RN) {
-        float t[HLP];
-        const float4* src = reinterpret_cast<const float4*>(s.h() + tid * HLP);
+    // then term + sum: IEEE addition commutes, so the order of the sum is what counts).
+    // All of the first wave runs it (the lanes past RN repeat the first RN), which then
+    // has the number of responses above the threshold and the largest in every lane.
+    int2 res = make_int2(0, 0);
+    if (tid < 64) {
+        const int p = tid % RN;
+        // the terms eight 16-byte loads at a time, the next eight on their way
+        constexpr int NQ = HLP / 4, CQ = 8;
+        float4 t[2][CQ];
+        const float4* src = reinterpret_cast<const float4*>(s.h() + p * HLP);
+        const auto fetch = [&](int g) {
 #pragma unroll
-        for (int q = 0; q < HLP / 4; ++q) {
-            const float4 v = src[q];
-            t[4 * q] = v.x; t[4 * q + 1] = v.y; t[4 * q + 2] = v.z; t[4 * q + 3] = v.w;
+            for (int q = 0; q < CQ; ++q)
+                if (g * CQ + q < NQ) t[g & 1][q] = src[g * CQ + q];
+        };
+        fetch(0);
+        float o = 0.f;
+#pragma unroll
+        for (int g = 0; g * CQ < NQ; ++g) {
+            fetch(g + 1);
+#pragma unroll
+            for (int q = 0; q < CQ; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int u = (g * CQ + q) * 4 + e;
+                    if (u < N::HL) {
+                        const float4 x = t[g & 1][q];
+                        const float y = e == 0 ? x.x : e == 1 ? x.y : e == 2 ? x.z : x.w;
+                        o = u == 0 ? y : y + o;
+                    }
+                }
         }
-        float o = t[0];
-#pragma unroll
-        for (int u = 1; u < N::HL; ++u) o = t[u] + o;
         float c = o + Wl[N::oOB];
         c = c * Wl[N::oOB + 1];
         c = rtanh(c);
         const float af = Wl[N::oOB + 2];
-        s.out()[tid] = (af == 0.f) ? (c + 1.f) * 0.5f : af * c;
+        const float d = (af == 0.f) ? (c + 1.f) * 0.5f : af * c;
+        if (out && tid < RN) out[tid] = d;
+        static_assert(RN == 16, "one row of lanes");
+        res.x = __popcll(__ballot(tid < RN && d > thr));
+        res.y = __float_as_int(row_max(fmaxf(d, -10.f)));
     }
-    __syncthreads();
     PHASE(PH_CHECK, PB + 5);
+    return res;
 }
 
 // Copies n floats of weights into LDS with all of a thread's loads in flight together
@@ -1660,15 +1761,9 @@ __device__ __forceinline__ void prepare_crop(const float* __restrict__ g, int gp
         if (tid < 64) {
             const int4 h = reinterpret_cast<const int4*>(s.hist())[tid];
             const int c0 = h.x, c1 = c0 + h.y, c2 = c1 + h.z, c3 = c2 + h.w;
-            int v = c3;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int a = __shfl_up(v, off, 64);
-                if (tid >= off) v += a;
-            }
-            const int b0 = v - c3;
+            const int b0 = wave_scan(c3) - c3;
             int4 cf = make_int4(b0 + c0, b0 + c1, b0 + c2, b0 + c3);
-            const float bmin = (float)__shfl(cf.x, 0, 64), bmax = (float)__shfl(cf.w, 63, 64);
+            const float bmin = (float)__builtin_amdgcn_readlane(cf.x, 0), bmax = (float)__builtin_amdgcn_readlane(cf.w, 63);
             if (bmin != bmax) {
                 const float delt = 255.f / (bmax - bmin);
                 cf.x = (int)(((float)cf.x - bmin) * delt + 0.5f);
@@ -1788,29 +1883,31 @@ __global__ void __launch_bounds__(CHECK_THREADS, 4) k_check(const float* __restr
         prepare_crop(g, gp, cr, P.equalize != 0, s, s_w, u, remap, tid, W2, W3, !staged);
         staged = true;
         PHASE(PH_CHECK, 1);
+        // the queue's next item is taken now, its latency behind the input's; s_item was
+        // read by every thread before the barriers of prepare_crop
+        int next = 0;
+        if (queue && threadIdx.x == 0) next = atomicAdd(queue, 1);
         write_input(s, u, remap, false, P.reflection != 0, tid);
+        if (queue && threadIdx.x == 0) s_item = next;
+        // the pixels alone stay in registers through stage 2, four to a word
+        constexpr int NP = (PER + 3) / 4;
+        uint32_t px[NP];
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            px[k] = u[4 * k] & 255u;
+#pragma unroll
+            for (int j = 1; j < 4; ++j)
+                if (4 * k + j < PER) px[k] |= (u[4 * k + j] & 255u) << (8 * j);
+        }
         PHASE(PH_CHECK, 2);
         PHASE_SET(PH_CHECK, 20, __smid());
         PHASE_SET(PH_CHECK, 21, item);
         PHASE_SET(PH_CHECK, 22, 0);
-        check_forward<Stage2, RP>(s.in, s, s.w, tid, MW2, s_w);
+        const int2 r2 = check_forward<Stage2, RP>(s.in, s, s.w, tid, P.t2, nullptr, MW2, s_w);
         if (tid == 0) {
-            float d[RN];
-#pragma unroll
-            for (int q = 0; q < RN / 4; ++q) {
-                const float4 v = reinterpret_cast<const float4*>(s.out())[q];
-                d[4 * q] = v.x; d[4 * q + 1] = v.y; d[4 * q + 2] = v.z; d[4 * q + 3] = v.w;
-            }
-            float m1 = -10.f;
-            int k1 = 0;
-#pragma unroll
-            for (int i = 0; i < RN; ++i) {
-                m1 = (m1 < d[i]) ? d[i] : m1;
-                if (d[i] > P.t2) k1++;
-            }
-            s2res[slot] = make_int2(k1, __float_as_int(m1));
-            if (hs2 && ci < hcap) hs2[slot] = make_int2(k1, __float_as_int(m1));
-            s_k1 = k1;
+            s2res[slot] = r2;
+            if (hs2 && ci < hcap) hs2[slot] = r2;
+            s_k1 = r2.x;
         }
         __syncthreads();
         const int k1 = s_k1;
@@ -1823,34 +1920,25 @@ __global__ void __launch_bounds__(CHECK_THREADS, 4) k_check(const float* __restr
                 if (hs3 && ci < hcap) hs3[slot] = make_int2(-1, __float_as_int(-10.f));
             }
         } else {
-        write_input(s, u, false, true, P.reflection != 0, tid);
-        PHASE(PH_CHECK, 16);
-        PHASE_SET(PH_CHECK, 22, 1);
-        check_forward<Stage3, RP>(s.in, s, s.w3, tid, MW3, s_w);
-        if (tid == 0) {
-            float d[RN];
+            int t3 = tid;                // opaque: the indices are formed again, not kept since prepare_crop
+            asm volatile("" : "+v"(t3));
 #pragma unroll
-            for (int q = 0; q < RN / 4; ++q) {
-                const float4 v = reinterpret_cast<const float4*>(s.out())[q];
-                d[4 * q] = v.x; d[4 * q + 1] = v.y; d[4 * q + 2] = v.z; d[4 * q + 3] = v.w;
+            for (int k = 0; k < PER; ++k) {
+                const int i = min(t3 + k * CHECK_THREADS, CW * CH - 1), iy = i / CW, ix = i - iy * CW;
+                u[k] = ((px[k / 4] >> (8 * (k & 3))) & 255u) | ((uint32_t)ix << 8) | ((uint32_t)iy << 16);
             }
-            float m2 = -10.f;
-            int k2 = 0;
-#pragma unroll
-            for (int i = 0; i < RN; ++i) {
-                m2 = (m2 < d[i]) ? d[i] : m2;
-                if (d[i] > P.t3) k2++;
+            write_input(s, u, false, true, P.reflection != 0, tid);
+            PHASE(PH_CHECK, 16);
+            PHASE_SET(PH_CHECK, 22, 1);
+            const int2 r3 = check_forward<Stage3, RP>(s.in, s, s.w3, tid, P.t3, nullptr, MW3, s_w);
+            if (tid == 0) {
+                s3res[slot] = r3;
+                if (hs3 && ci < hcap) hs3[slot] = r3;
             }
-            s3res[slot] = make_int2(k2, __float_as_int(m2));
-            if (hs3 && ci < hcap) hs3[slot] = make_int2(k2, __float_as_int(m2));
-        }
         }
         PHASE(PH_CHECK, 15);
-        // the next item: every thread reads it after the barrier, and the previous item's
-        // last LDS reads are done before it is written
+        // the next item, when this one's last LDS reads are done
         if (queue) {
-            __syncthreads();
-            if (threadIdx.x == 0) s_item = atomicAdd(queue, 1);
             __syncthreads();
             item = s_item;
         } else {
@@ -2272,8 +2360,7 @@ __global__ void __launch_bounds__(CHECK_THREADS, 4) k_net23(const float* __restr
     stage_weights<N::SIZE>(s.w, W, tid);
     for (int i = tid; i < IW * IH; i += CHECK_THREADS) s.in[i] = src[i];
     __syncthreads();
-    check_forward<N, RP>(s.in, s, s.w, tid, MW, s_red);
-    if (tid < RN) out[(size_t)blockIdx.x * RN + tid] = s.out()[tid];
+    check_forward<N, RP>(s.in, s, s.w, tid, 0.f, out + (size_t)blockIdx.x * RN, MW, s_red);
 }
 
 // The landmarks network on one 49x51 input (tests).
