@@ -26,14 +26,26 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("CCNN_OFFLOAD_ARCH", "gfx950")
 
 
-def gen_models(path):
-    lines = ["// generated from compactcnncascade_amd/models by build.py", "#include <cstddef>",
-             "namespace ccnn {"]
+def _write(path, lines):
+    text = "\n".join(["// generated from compactcnncascade_amd/models by build.py"] + lines) + "\n"
+    old = open(path).read() if os.path.exists(path) else None
+    if old != text:
+        with open(path, "w") as f:
+            f.write(text)
+
+
+def gen_models(path, header):
+    """The model files as byte arrays: the three cascade networks in `header` (constants of
+    the kernels that carry weights as literals, ccnn_weights.h), all of them behind
+    embedded_model in `path`."""
+    arrays = []
     for i, name in enumerate(MODELS):
         with open(os.path.join(PKG, "models", name), "rb") as f:
             data = f.read()
         body = ",".join(str(b) for b in data)
-        lines.append("static const unsigned char k_model%d[%d] = {%s};" % (i, len(data), body))
+        arrays.append("constexpr unsigned char k_model%d[%d] = {%s};" % (i, len(data), body))
+    _write(header, ["#pragma once", "namespace ccnn {"] + arrays[:3] + ["}  // namespace ccnn"])
+    lines = ["#include <cstddef>", '#include "%s"' % os.path.basename(header), "namespace ccnn {"] + arrays[3:]
     lines.append("void embedded_model(int stage, const unsigned char** bytes, size_t* n)")
     lines.append("{")
     for i in range(len(MODELS)):
@@ -41,11 +53,7 @@ def gen_models(path):
     lines.append("    *bytes = nullptr; *n = 0;")
     lines.append("}")
     lines.append("}  // namespace ccnn")
-    text = "\n".join(lines) + "\n"
-    old = open(path).read() if os.path.exists(path) else None
-    if old != text:
-        with open(path, "w") as f:
-            f.write(text)
+    _write(path, lines)
 
 
 def build(verbose=True, phase_stamps=False):
@@ -53,7 +61,7 @@ def build(verbose=True, phase_stamps=False):
     library with the kernels' phase timestamps, for ccnn_phase_stamps)."""
     os.makedirs(BUILD, exist_ok=True)
     models_cpp = os.path.join(BUILD, "ccnn_models.cpp")
-    gen_models(models_cpp)
+    gen_models(models_cpp, os.path.join(BUILD, "ccnn_model_bytes.h"))
     srcs = [os.path.join(CSRC, s) for s in SOURCES] + [models_cpp]
     lib = PHASES_LIB if phase_stamps else LIB
     tmp = lib + ".tmp"
@@ -65,7 +73,7 @@ def build(verbose=True, phase_stamps=False):
            "-Wno-unused-command-line-argument",
            # every symbol the library references must resolve at link time
            "-Wl,-z,defs",
-           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
+           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-I" + BUILD,
            "-o", tmp] + (["-DCCNN_PHASE_STAMPS"] if phase_stamps else []) + srcs
     if verbose:
         print(" ".join(cmd), flush=True)

@@ -28,6 +28,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 #include "ccnn_internal.h"
+#include "ccnn_weights.h"
 
 #include <type_traits>
 
@@ -107,8 +108,10 @@ __device__ __forceinline__ float rtanh(float c)
     const float a = 1.41645f;
     const float den = ((fabsf(c) + c * c) + a * c * c * c * c) + 1.f;
     const float t = 1.f - (IEEE_DIV ? 1.f / den : recip_ge1(den));
-    // the reference multiplies by sgn = -1 or 1, which is the negation or t itself
-    return c < 0.f ? -t : t;
+    // the reference multiplies by sgn = -1 or 1 (c < 0 or not): t >= 0 with the sign of c,
+    // where c + 0 has the sign + for both zeros. One v_bfi_b32 (4 clocks) and an add (2);
+    // a v_cndmask_b32 whose condition was not written right before it takes 16
+    return __builtin_copysignf(t, c + 0.f);
 }
 
 __device__ __forceinline__ float lrelu_bn(float conv, const float* __restrict__ p, int m, int M)
@@ -401,6 +404,13 @@ __global__ void __launch_bounds__(256) k_level(const float* __restrict__ g, int 
 // Each pooled L1 position depends only on the level samples at (2X..2X+4, 2Y..2Y+4),
 // so the split computes the same values as one fused pass without recomputing the
 // L1 halo that neighbouring response tiles share.
+// What bounds them is VALU issue. In the exact form the weights are literals
+// (ccnn_weights.h): as SGPR operands the L1 and L2 products held the stream to 0.32
+// instructions a clock of 0.44, and the tail's weights in LDS (26.9 KB a workgroup more to
+// fetch and read) took 93 VGPRs; now 75 and six workgroups a CU instead of five. 64
+// frames of 1920x1080: k_stage1_l1 923 -> 836 us, k_stage1 1227 -> 1078 us; one frame:
+// k_stage1 28.6 -> 23.5 us. The FP16 form keeps its weights in memory: its products take
+// an issue slot of 4 clocks whatever their operands are.
 // ---------------------------------------------------------------------------------
 namespace s1 {
 using N = Stage1;
@@ -575,8 +585,7 @@ __global__ void __launch_bounds__(S1A_THREADS) k_stage1_l1(const float* __restri
 
     // L1: conv_4x4 chains + lrelu_bn_max for every map, then the sums feeding L2
     // (add / add2, cnnpp_cplusplus.cpp:916-950; wiring cnn_simd_cntk.cpp:705-725)
-    const float* k1 = W + N::oK1;
-    const float* b1 = W + N::oB1;
+    [[maybe_unused]] const float* b1 = W + N::oB1;
     const size_t plane = (size_t)L.s1_w * L.s1_h;
     float* out = s1buf + L.s1_off;
     // the positions responses inside the map read (vx x vy of the tile; fewer at the
@@ -625,20 +634,7 @@ __global__ void __launch_bounds__(S1A_THREADS) k_stage1_l1(const float* __restri
                 pm[m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
             }
         } else {
-#pragma unroll
-        for (int m = 0; m < N::M1; ++m) {
-            const float* k = k1 + m * 16;
-            float a[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int dx = q & 1, dy = q >> 1;
-                float acc = win[dy][dx] * k[0];
-#pragma unroll
-                for (int j = 1; j < 16; ++j) acc = acc + win[dy + (j >> 2)][dx + (j & 3)] * k[j];
-                a[q] = lrelu_bn(acc, b1, m, N::M1);
-            }
-            pm[m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
-        }
+        static_for<N::M1>([&](auto m) { pm[m] = conv4_act_pool<N, N::oK1 + m * 16, N::oB1, N::M1, m>(win); });
         }
         float* o = out + (size_t)Y * L.s1_w + X;
         o[0] = pm[0] + pm[1];
@@ -662,15 +658,16 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     constexpr int P1W = G::P1W, P1H = G::P1H, P2W = G::P2W, P1N = G::P1N, P2N = G::P2N;
     static_assert(TX * TY <= S1_THREADS, "one response value per thread");
     __shared__ __align__(16) float s_s1[N::M1 * P1N];     // L1 sums; later the L2 sums and tail weights
-    // the L3, hidden- and output-layer weights, which the per-response tail reads from
-    // LDS; fetched into registers now, stored over the consumed L2 maps later
+    // FP16 path: the L3, hidden- and output-layer weights, which the per-response tail
+    // reads from LDS; fetched into registers now, stored over the consumed L2 maps later
     constexpr int WT = N::SIZE - N::oK3, WPER = (WT + S1_THREADS - 1) / S1_THREADS;
 
-
     const int tid = threadIdx.x;
-    float wt[WPER];
+    [[maybe_unused]] float wt[WPER];
+    if constexpr (H) {
 #pragma unroll
-    for (int k = 0; k < WPER; ++k) wt[k] = W[N::oK3 + min(tid + k * S1_THREADS, WT - 1)];
+        for (int k = 0; k < WPER; ++k) wt[k] = W[N::oK3 + min(tid + k * S1_THREADS, WT - 1)];
+    }
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     PHASE_CLEAR();
     PHASE(PH_STAGE1, 0);
@@ -735,8 +732,7 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     // L2, one pooled L2 position per thread: the eight maps (two conv_3x3 chains per L1
     // sum + lrelu_bn_max), then their neighbour sums, held in registers until every thread
     // has read the L1 sums and then written over them
-    const float* k2 = W + N::oK2;
-    const float* b2 = W + N::oB2;
+    [[maybe_unused]] const float* b2 = W + N::oB2;
     constexpr int RP = (P2W * G::P2H + S1_THREADS - 1) / S1_THREADS;   // positions per thread
     float sv[RP][N::M2];
 #pragma unroll
@@ -745,8 +741,7 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
         if (r >= nq) break;
         const int qy = (int)(((float)r + 0.5f) * rqw), qx = r - qy * qw;
         float v[N::M2];
-#pragma unroll
-        for (int i = 0; i < N::M1; ++i) {
+        static_for<N::M1>([&](auto i) {
             const float* src = s_s1 + i * P1N + (2 * qy) * P1W + 2 * qx;
             float win[4][4];
 #pragma unroll
@@ -782,23 +777,12 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
                     v[m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
                 }
             } else {
-#pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    const int m = 2 * i + half;
-                    const float* kk = k2 + m * 9;
-                    float a[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int dx = q & 1, dy = q >> 1;
-                        float acc = win[dy][dx] * kk[0];
-#pragma unroll
-                        for (int j = 1; j < 9; ++j) acc = acc + win[dy + j / 3][dx + j % 3] * kk[j];
-                        a[q] = lrelu_bn(acc, b2, m, N::M2);
-                    }
-                    v[m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
-                }
+                static_for<2>([&](auto half) {
+                    constexpr int m = 2 * i + half;
+                    v[m] = conv3_act_pool<N, N::oK2 + m * 9, N::oB2, N::M2, m>(win);
+                });
             }
-        }
+        });
         sv[k][0] = v[0] + v[1];
 #pragma unroll
         for (int i = 1; i < N::M2 - 1; ++i) sv[k][i] = v[i - 1] + v[i] + v[i + 1];
@@ -809,7 +793,7 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     // the L2 sums over the (consumed) L1 sums, with rows P2S floats apart: an odd multiple
     // of 8, so that the rows of an 8 x 8 block of responses (below) start in distinct
     // groups of 8 LDS banks and the L3 window reads of a wave are free of bank conflicts;
-    // the tail weights after them
+    // on the FP16 path the tail weights after them
     constexpr int P2S = (P2W + 7) / 16 * 16 + 8, P2NS = P2S * G::P2H;
     float* s_s2 = s_s1;
 #pragma unroll
@@ -821,15 +805,15 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
 #pragma unroll
         for (int m = 0; m < N::M2; ++m) s_s2[m * P2NS + ps] = sv[k][m];
     }
-    float* s_wt = s_s1 + N::M2 * P2NS;
+    [[maybe_unused]] float* s_wt = s_s1 + N::M2 * P2NS;
     static_assert(P2S >= P2W && N::M2 * P2NS + WT + Stage1H::SIZE <= N::M1 * P1N,
                   "L2 sums and tail weights fit in the L1-sum space");
-#pragma unroll
-    for (int k = 0; k < WPER; ++k)
-        if (tid + k * S1_THREADS < WT) s_wt[tid + k * S1_THREADS] = wt[k];
-    // FP16 path: the L3 and hidden-layer tap pairs follow the FP32 tail weights in LDS
-    uint32_t* s_wh = reinterpret_cast<uint32_t*>(s_wt + WT);
+    // the L3 and hidden-layer tap pairs follow the FP32 tail weights in LDS
+    [[maybe_unused]] uint32_t* s_wh = reinterpret_cast<uint32_t*>(s_wt + WT);
     if constexpr (H) {
+#pragma unroll
+        for (int k = 0; k < WPER; ++k)
+            if (tid + k * S1_THREADS < WT) s_wt[tid + k * S1_THREADS] = wt[k];
         const uint32_t* src = reinterpret_cast<const uint32_t*>(W + N::SIZE) + Stage1H::oL3;
         for (int k = tid; k < Stage1H::SIZE - Stage1H::oL3; k += S1_THREADS) s_wh[k] = src[k];
     }
@@ -853,12 +837,10 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
         oy = (int)(((float)tid + 0.5f) * rvw);
         ox = tid - oy * vw;
     }
-    const float* Wt = s_wt - N::oK3;   // indexed with the offsets into W
-    const float* k3 = Wt + N::oK3;
-    const float* b3 = Wt + N::oB3;
+    const float* Wt = H ? s_wt - N::oK3 : W;   // indexed with the offsets into W
+    [[maybe_unused]] const float* b3 = Wt + N::oB3;
     float a3[N::M3];
-#pragma unroll
-    for (int i = 0; i < N::M2; ++i) {
+    static_for<N::M2>([&](auto i) {
         const float* src = s_s2 + i * P2NS + oy * P2S + ox;
         float win[N::K3H][N::K3W];
 #pragma unroll
@@ -885,23 +867,21 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
                 }
                 a3[m] = lrelu_bn_fma(d, b3, m, N::M3);
             }
-            continue;
+        } else {
+            static_for<2>([&](auto half) {
+                constexpr int m = 2 * i + half, k = N::oK3 + m * N::K3W * N::K3H;
+                float d = 0.f;
+                static_for<N::K3H>([&](auto r) {
+                    float rs = win[r][0] * weight_v<N, k + r * N::K3W>;
+                    static_for<N::K3W - 1>([&](auto c) {
+                        rs = rs + win[r][c + 1] * weight_v<N, k + r * N::K3W + c + 1>;
+                    });
+                    d = (r == 0) ? rs : d + rs;
+                });
+                a3[m] = lrelu_bn_w<N, N::oB3, N::M3, m>(d);
+            });
         }
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int m = 2 * i + half;
-            const float* k = k3 + m * N::K3W * N::K3H;
-            float d = 0.f;
-#pragma unroll
-            for (int r = 0; r < N::K3H; ++r) {
-                float rs = win[r][0] * k[r * N::K3W];
-#pragma unroll
-                for (int c = 1; c < N::K3W; ++c) rs = rs + win[r][c] * k[r * N::K3W + c];
-                d = (r == 0) ? rs : d + rs;
-            }
-            a3[m] = lrelu_bn(d, b3, m, N::M3);
-        }
-    }
+    });
     // hidden layer: mulCN_add_tanhW (cnnpp_cplusplus.cpp:646-672, loop cnn_simd_cntk.cpp:874-883)
     float hv[N::HL];
     if constexpr (H) {
@@ -921,19 +901,16 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
                 hv[u] = __builtin_fmaf(Wt[N::oHBW + tt], __builtin_fmaf(c, 0.5f, 0.5f), Wt[N::oHBB + tt]);
             }
     } else {
-#pragma unroll
-    for (int gi = 0; gi < N::HLG; ++gi)
-#pragma unroll
-        for (int tt = 0; tt < N::HLS; ++tt) {
-            const int u = N::HLS * gi + tt;
-            float c = Wt[N::oHB + u];
-#pragma unroll
-            for (int j = 0; j < N::HLN; ++j) c = c + a3[gi + j] * Wt[N::oHW + u * N::HLN + j];
-            c = c * Wt[N::oHT + gi];
-            c = rtanh(c);
+        static_for<N::HL>([&](auto u) {
+            constexpr int gi = u / N::HLS, tt = u % N::HLS;
+            float c = weight_v<N, N::oHB + u> + a3[gi] * weight_v<N, N::oHW + u * N::HLN>;
+            static_for<N::HLN - 1>([&](auto j) {
+                c = c + a3[gi + j + 1] * weight_v<N, N::oHW + u * N::HLN + j + 1>;
+            });
+            c = rtanh(c * weight_v<N, N::oHT + gi>);
             c = (c + 1.f) * 0.5f;
-            hv[u] = Wt[N::oHBW + tt] * c + Wt[N::oHBB + tt];
-        }
+            hv[u] = weight_v<N, N::oHBW + tt> * c + weight_v<N, N::oHBB + tt>;
+        });
     }
     // output layer: mulC / mulC1_add / tanhW (cnnpp_cplusplus.cpp:952-984, 673-690)
     float o = 0.f;
