@@ -516,8 +516,8 @@ __global__ void __launch_bounds__(S1A_THREADS) k_stage1_l1(const float* __restri
     // store. The three columns past the groups are left to one sample per thread. (With
     // the samples numbered through, each looked up both tables: 27 instructions a sample,
     // among them multiplies of 4 clocks for its row and column; now 11 of 2 clocks. 64 1080p
-    // frames: 836 -> 804 us; FP16 form, mixed batch: 890 -> 832 us; one frame: 23.7 -> 22.8
-    // us.) Rows go in batches so that their loads are in flight together.
+    // frames: 836 -> 804 us; FP16 form, mixed batch: 890 -> 832 us; one frame: 23.7 -> 22.8 us.) Rows go in batches so that their loads are in
+    // flight together.
     {
         constexpr int NE = AW - 64 * NCG;
         static_assert(NE * AH <= S1A_THREADS, "one remainder sample per thread");
@@ -1419,6 +1419,7 @@ __device__ __forceinline__ int2 check_forward(const float* __restrict__ in, ChkS
     constexpr unsigned WAVES = CHECK_THREADS / 64, PW = P1N / WAVES, PREM = PW % 64;
     static_assert(P1N % WAVES == 0 && PREM == 4 && N::M1 == 6, "remainder: 4 positions x 4 quads x 3 map pairs");
     const unsigned wave = ut >> 6, lane = ut & 63u;
+#pragma unroll 1
     for (unsigned w0 = lane; w0 < PW - PREM; w0 += 64) {
         const unsigned p = wave * PW + w0;
         const unsigned py = p / P1W, px = p - py * P1W;
@@ -1428,20 +1429,7 @@ __device__ __forceinline__ int2 check_forward(const float* __restrict__ in, ChkS
 #pragma unroll
             for (int c = 0; c < 5; ++c) win[r][c] = in[(2 * py + r) * IW + 2 * px + c];
         float pm[N::M1];
-#pragma unroll
-        for (int m = 0; m < N::M1; ++m) {
-            const float* k = Wl + N::oK1 + m * 16;
-            float a[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int dx = q & 1, dy = q >> 1;
-                float acc = win[dy][dx] * k[0];
-#pragma unroll
-                for (int j = 1; j < 16; ++j) acc = acc + win[dy + (j >> 2)][dx + (j & 3)] * k[j];
-                a[q] = lrelu_bn(acc, Wl + N::oB1, m, N::M1);
-            }
-            pm[m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
-        }
+        static_for<N::M1>([&](auto m) { pm[m] = conv4_act_pool<N, N::oK1 + m * 16, N::oB1, N::M1, m>(win); });
         s.s1[p] = pm[0] + pm[1];
 #pragma unroll
         for (int i = 1; i < N::M1 - 1; ++i) s.s1[i * P1N + p] = pm[i - 1] + pm[i] + pm[i + 1];
@@ -1480,31 +1468,27 @@ __device__ __forceinline__ int2 check_forward(const float* __restrict__ in, ChkS
     }
     __syncthreads();
     PHASE(PH_CHECK, PB + 0);
-    // L2
-    for (unsigned it = ut; it < N::M1 * P2N; it += CHECK_THREADS) {
-        const unsigned i = it / P2N, p = it - i * P2N;
+    // L2: a wave takes one of a sum's two halves of positions (64 and the rest), so that its
+    // maps, and with them the literal weights, are the same in all lanes
+    static_assert(P2N > 64 && P2N <= 128 && 2 * N::M1 % WAVES == 0, "two waves of positions a sum");
+#pragma unroll 1
+    for (unsigned k = __builtin_amdgcn_readfirstlane(wave); k < 2 * N::M1; k += WAVES) {
+        const unsigned sum = k >> 1, p = (k & 1u) * 64 + lane;
+        if (p >= P2N) continue;
         const unsigned qy = p / P2W, qx = p - qy * P2W;
-        const float* src = s.s1 + i * P1N + (2 * qy) * P1W + 2 * qx;
+        const float* src = s.s1 + sum * P1N + (2 * qy) * P1W + 2 * qx;
         float win[4][4];
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
             for (int c = 0; c < 4; ++c) win[r][c] = src[r * P1W + c];
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int m = 2 * i + half;
-            const float* k = Wl + N::oK2 + m * 9;
-            float a[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int dx = q & 1, dy = q >> 1;
-                float acc = win[dy][dx] * k[0];
-#pragma unroll
-                for (int j = 1; j < 9; ++j) acc = acc + win[dy + j / 3][dx + j % 3] * k[j];
-                a[q] = lrelu_bn(acc, Wl + N::oB2, m, N::M2);
-            }
-            s.p2()[m * P2N + p] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
-        }
+        static_for<N::M1>([&](auto i) {
+            if (sum != i) return;
+            static_for<2>([&](auto half) {
+                constexpr int m = 2 * i + half;
+                s.p2()[m * P2N + p] = conv3_act_pool<N, N::oK2 + m * 9, N::oB2, N::M2, m>(win);
+            });
+        });
     }
     __syncthreads();
     PHASE(PH_CHECK, PB + 1);
