@@ -75,12 +75,14 @@ __shared__ unsigned long long s_phase[PHASE_SLOTS];
     } while (0)
 #endif
 #define PHASE(kern, slot) PHASE_SET(kern, slot, wall_clock64())
-// the stamps cost k_stage1 registers; the profiling build keeps its occupancy at the
-// default build's 5 waves per SIMD so that the stamped phases are those of the product
+// k_stage1's waves per SIMD (H: its FP16 form). Exact: eight, which costs 4 spilled VGPRs and
+// is still faster than the seven of the compiler's choice (64 1080p frames 982 us against
+// 1003); FP16: six, what its registers allow. The stamps cost registers; the profiling
+// build runs six of either.
 #ifdef CCNN_PHASE_STAMPS
-#define S1_WAVES __attribute__((amdgpu_waves_per_eu(5)))
+#define S1_WAVES __attribute__((amdgpu_waves_per_eu(6)))
 #else
-#define S1_WAVES
+#define S1_WAVES __attribute__((amdgpu_waves_per_eu(H ? 6 : 8)))
 #endif
 enum { PH_CHECK = 0, PH_STAGE1 = 1 };
 
@@ -407,11 +409,13 @@ __global__ void __launch_bounds__(256) k_level(const float* __restrict__ g, int 
 // L1 halo that neighbouring response tiles share.
 // What bounds them is VALU issue. In the exact form the weights are literals
 // (ccnn_weights.h): as SGPR operands the L1 and L2 products held the stream to 0.32
-// instructions a clock of 0.44, and the tail's weights in LDS (26.9 KB a workgroup more to
-// fetch and read) took 93 VGPRs; now 75 and six workgroups a CU instead of five. 64
+// instructions a clock of 0.44, and the tail's weights took LDS reads and 93 VGPRs. 64
 // frames of 1920x1080: k_stage1_l1 923 -> 836 us, k_stage1 1227 -> 1078 us; one frame:
-// k_stage1 28.6 -> 23.5 us. The FP16 form keeps its weights in memory: its products take
-// an issue slot of 4 clocks whatever their operands are.
+// k_stage1 28.6 -> 23.5 us. Two planes of L1 sums at a time in LDS, the other two on their
+// way meanwhile, make room for eight workgroups on a CU instead of six: k_stage1 1051 -> 982
+// us for the 64 frames, 1923 -> 1714 us for a 4800x2400 frame in 91 levels, 22.9 -> 22.0 us
+// for one 1080p frame. The FP16 form keeps its weights in memory (its products take
+// an issue slot of 4 clocks whatever their operands are) and all its planes in LDS.
 // ---------------------------------------------------------------------------------
 namespace s1 {
 using N = Stage1;
@@ -677,7 +681,16 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     using G = s1::RespGeo<TX, TY>;
     constexpr int P1W = G::P1W, P1H = G::P1H, P2W = G::P2W, P1N = G::P1N, P2N = G::P2N;
     static_assert(TX * TY <= S1_THREADS, "one response value per thread");
-    __shared__ __align__(16) float s_s1[N::M1 * P1N];     // L1 sums; later the L2 sums and tail weights
+    // rows of the L2 sums P2S floats apart: an odd multiple of 8, so that the rows of an
+    // 8 x 8 block of responses (below) start in distinct groups of 8 LDS banks and the L3
+    // window reads of a wave are free of bank conflicts
+    constexpr int P2S = (P2W + 7) / 16 * 16 + 8, P2NS = P2S * G::P2H;
+    static_assert(P2S >= P2W, "rows of L2 sums");
+    // L1 sums, PL planes at a time (exact: two, FP16: all); later the L2 sums and, on the FP16
+    // path, the tail weights. With 15.4 KB instead of 26.9 KB and 64 VGPRs eight workgroups
+    // run on a CU instead of six
+    constexpr int PL = H ? N::M1 : 2, S1N = PL * P1N > N::M2 * P2NS ? PL * P1N : N::M2 * P2NS;
+    __shared__ __align__(16) float s_s1[S1N];
     // FP16 path: the L3, hidden- and output-layer weights, which the per-response tail
     // reads from LDS; fetched into registers now, stored over the consumed L2 maps later
     constexpr int WT = N::SIZE - N::oK3, WPER = (WT + S1_THREADS - 1) / S1_THREADS;
@@ -725,109 +738,117 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     // the tile's L1 sums: rows 2*oy0 .. +P1H, columns 2*ox0 .. +P1W of each plane
     // (inside the planes: s1_w = 2*TX*tiles_x + 8, s1_h = 2*TY*tiles_y + 10). Every
     // plane row and level offset is a multiple of 8 floats and 2*ox0 of 32, so the rows
-    // are copied as float4; the M1 planes stack as M1*P1H rows of the tile window.
-    {
-        static_assert(P1W % 4 == 0 && (2 * TX) % 4 == 0, "float4 rows");
-        constexpr int RQ = P1W / 4, NQ = N::M1 * P1H * RQ;
-        constexpr int PER = (NQ + S1_THREADS - 1) / S1_THREADS, B = PER;   // one batch
+    // are copied as float4; the PL planes stack as PL*P1H rows of the tile window. On the
+    // exact path the second half of the planes is on its way while the first is in use.
+    static_assert(P1W % 4 == 0 && (2 * TX) % 4 == 0, "float4 rows");
+    constexpr int RQ = P1W / 4, NQ = PL * P1H * RQ;
+    constexpr int PER = (NQ + S1_THREADS - 1) / S1_THREADS;
+    typedef float f4_t __attribute__((ext_vector_type(4)));
+    f4_t fetched[PER];
+    const auto fetch = [&](int plane0) {
         const uint32_t plane = (uint32_t)L.s1_w * L.s1_h;
-        const float* src = s1buf + L.s1_off + (size_t)(2 * oy0) * L.s1_w + 2 * ox0;
-        float4 v[B];
-#pragma unroll
-        for (int k = 0; k < B; ++k) {
+        const float* src = s1buf + L.s1_off + (size_t)(2 * oy0) * L.s1_w + 2 * ox0 + (size_t)plane0 * plane;
+        static_for<PER>([&](auto k) {
             const int i = min(tid + k * S1_THREADS, NQ - 1);
             const int row = i / RQ, q = i - row * RQ;       // row of the stacked planes
             const int m = row / P1H, py = row - m * P1H;
-            v[k] = *reinterpret_cast<const float4*>(src + m * plane + (uint32_t)py * L.s1_w + 4 * q);
-        }
-#pragma unroll
-        for (int k = 0; k < B; ++k) {
+            fetched[k] = *reinterpret_cast<const f4_t*>(src + m * plane + (uint32_t)py * L.s1_w + 4 * q);
+        });
+    };
+    const auto put = [&]() {
+        static_for<PER>([&](auto k) {
             const int i = tid + k * S1_THREADS;
-            if (i < NQ) *reinterpret_cast<float4*>(s_s1 + 4 * i) = v[k];
-        }
-    }
+            if (i < NQ) *reinterpret_cast<f4_t*>(s_s1 + 4 * i) = fetched[k];
+        });
+    };
+    fetch(0);
+    put();
     __syncthreads();
     PHASE(PH_STAGE1, 1);
 
     // L2, one pooled L2 position per thread: the eight maps (two conv_3x3 chains per L1
-    // sum + lrelu_bn_max), then their neighbour sums, held in registers until every thread
-    // has read the L1 sums and then written over them
+    // sum + lrelu_bn_max), held in registers until every thread has read the L1 sums, whose
+    // place their neighbour sums then take
     [[maybe_unused]] const float* b2 = W + N::oB2;
     constexpr int RP = (P2W * G::P2H + S1_THREADS - 1) / S1_THREADS;   // positions per thread
     float sv[RP][N::M2];
+    // the maps of the sums in LDS, from sum I0 of the network on
+    const auto l2 = [&](auto first) {
+        constexpr int I0 = first;
+        static_for<RP>([&](auto k) {
+            const int r = tid + k * S1_THREADS;
+            if (r >= nq) return;
+            const int qy = (int)(((float)r + 0.5f) * rqw), qx = r - qy * qw;
+            static_for<PL>([&](auto local) {
+                constexpr int i = I0 + local;
+                const float* src = s_s1 + local * P1N + (2 * qy) * P1W + 2 * qx;
+                float win[4][4];
 #pragma unroll
-    for (int k = 0; k < RP; ++k) {
-        const int r = tid + k * S1_THREADS;
-        if (r >= nq) break;
-        const int qy = (int)(((float)r + 0.5f) * rqw), qx = r - qy * qw;
-        float v[N::M2];
-        static_for<N::M1>([&](auto i) {
-            const float* src = s_s1 + i * P1N + (2 * qy) * P1W + 2 * qx;
-            float win[4][4];
+                for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+                    for (int c = 0; c < 4; ++c) win[r][c] = src[r * P1W + c];
+                if constexpr (H) {
+                    // pairs (c, c+1) of each window row, and (c3, 0) for the last tap of the
+                    // right-hand quads; per map and row the tap pairs (k0, k1), (k2, 0)
+                    h2_t hp[4][3], hz[4];
 #pragma unroll
-                for (int c = 0; c < 4; ++c) win[r][c] = src[r * P1W + c];
-            if constexpr (H) {
-                // pairs (c, c+1) of each window row, and (c3, 0) for the last tap of the
-                // right-hand quads; per map and row the tap pairs (k0, k1), (k2, 0)
-                h2_t hp[4][3], hz[4];
+                    for (int r = 0; r < 4; ++r) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) hp[r][c] = pk16(win[r][c], win[r][c + 1]);
-                    hz[r] = pk16(win[r][3], 0.f);
-                }
-                const uint32_t* kh = reinterpret_cast<const uint32_t*>(W + N::SIZE) + Stage1H::oL2;
-#pragma unroll
-                for (int half = 0; half < 2; ++half) {
-                    const int m = 2 * i + half;
-                    float a[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int dx = q & 1, dy = q >> 1;
-                        float acc = 0.f;
-#pragma unroll
-                        for (int r = 0; r < 3; ++r) {
-                            acc = dot2(hp[dy + r][dx], as_h2(kh[m * 6 + 2 * r]), acc);
-                            acc = dot2(dx ? hz[dy + r] : hp[dy + r][2], as_h2(kh[m * 6 + 2 * r + 1]), acc);
-                        }
-                        a[q] = lrelu_bn_fma(acc, b2, m, N::M2);
+                        for (int c = 0; c < 3; ++c) hp[r][c] = pk16(win[r][c], win[r][c + 1]);
+                        hz[r] = pk16(win[r][3], 0.f);
                     }
-                    v[m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
-                }
-            } else {
-                static_for<2>([&](auto half) {
-                    constexpr int m = 2 * i + half;
-                    v[m] = conv3_act_pool<N, N::oK2 + m * 9, N::oB2, N::M2, m>(win);
-                });
-            }
-        });
-        sv[k][0] = v[0] + v[1];
+                    const uint32_t* kh = reinterpret_cast<const uint32_t*>(W + N::SIZE) + Stage1H::oL2;
 #pragma unroll
-        for (int i = 1; i < N::M2 - 1; ++i) sv[k][i] = v[i - 1] + v[i] + v[i + 1];
-        sv[k][N::M2 - 1] = v[N::M2 - 2] + v[N::M2 - 1];
+                    for (int half = 0; half < 2; ++half) {
+                        const int m = 2 * i + half;
+                        float a[4];
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const int dx = q & 1, dy = q >> 1;
+                            float acc = 0.f;
+#pragma unroll
+                            for (int r = 0; r < 3; ++r) {
+                                acc = dot2(hp[dy + r][dx], as_h2(kh[m * 6 + 2 * r]), acc);
+                                acc = dot2(dx ? hz[dy + r] : hp[dy + r][2], as_h2(kh[m * 6 + 2 * r + 1]), acc);
+                            }
+                            a[q] = lrelu_bn_fma(acc, b2, m, N::M2);
+                        }
+                        sv[k][m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
+                    }
+                } else {
+                    static_for<2>([&](auto half) {
+                        constexpr int m = 2 * i + half;
+                        sv[k][m] = conv3_act_pool<N, N::oK2 + m * 9, N::oB2, N::M2, m>(win);
+                    });
+                }
+            });
+        });
+    };
+    l2(std::integral_constant<int, 0>{});
+    if constexpr (!H) {
+        fetch(2);
+        __syncthreads();
+        put();
+        __syncthreads();
+        l2(std::integral_constant<int, 2>{});
     }
     __syncthreads();
     PHASE(PH_STAGE1, 2);
-    // the L2 sums over the (consumed) L1 sums, with rows P2S floats apart: an odd multiple
-    // of 8, so that the rows of an 8 x 8 block of responses (below) start in distinct
-    // groups of 8 LDS banks and the L3 window reads of a wave are free of bank conflicts;
-    // on the FP16 path the tail weights after them
-    constexpr int P2S = (P2W + 7) / 16 * 16 + 8, P2NS = P2S * G::P2H;
+    // the L2 sums over the (consumed) L1 sums; on the FP16 path the tail weights after them
     float* s_s2 = s_s1;
-#pragma unroll
-    for (int k = 0; k < RP; ++k) {
+    static_for<RP>([&](auto k) {
         const int r = tid + k * S1_THREADS;
-        if (r >= nq) break;
+        if (r >= nq) return;
         const int qy = (int)(((float)r + 0.5f) * rqw), qx = r - qy * qw;
         const int ps = qy * P2S + qx;
+        const auto& v = sv[k];
+        s_s2[ps] = v[0] + v[1];
 #pragma unroll
-        for (int m = 0; m < N::M2; ++m) s_s2[m * P2NS + ps] = sv[k][m];
-    }
+        for (int m = 1; m < N::M2 - 1; ++m) s_s2[m * P2NS + ps] = v[m - 1] + v[m] + v[m + 1];
+        s_s2[(N::M2 - 1) * P2NS + ps] = v[N::M2 - 2] + v[N::M2 - 1];
+    });
     [[maybe_unused]] float* s_wt = s_s1 + N::M2 * P2NS;
-    static_assert(P2S >= P2W && N::M2 * P2NS + WT + Stage1H::SIZE <= N::M1 * P1N,
-                  "L2 sums and tail weights fit in the L1-sum space");
+    static_assert(!H || N::M2 * P2NS + WT + Stage1H::SIZE <= S1N, "L2 sums and tail weights fit in the L1-sum space");
     // the L3 and hidden-layer tap pairs follow the FP32 tail weights in LDS
     [[maybe_unused]] uint32_t* s_wh = reinterpret_cast<uint32_t*>(s_wt + WT);
     if constexpr (H) {
