@@ -343,7 +343,7 @@ int Detector::run_batch(const std::vector<BatchFrame>& seg, bool device_ptr, std
         q0 += (long long)F.qw * F.h;
         const uintptr_t al = F.ch == 4 ? 16 : 4;
         F.aligned = (((uintptr_t)F.src % al) == 0 && (uintptr_t)F.step % al == 0 ? 1 : 0) |
-                    (((uintptr_t)F.src % 16) == 0 && (uintptr_t)F.step % 16 == 0 ? 2 : 0);
+                    (((uintptr_t)F.src % 4) == 0 && (uintptr_t)F.step % 4 == 0 ? 2 : 0);
         B.h_ftab[fi] = F;
     }
     HIP_OK(hipMemcpyAsync(B.d_ftab, B.h_ftab, sizeof(FrameDesc) * nf, hipMemcpyHostToDevice, B.st));
