@@ -75,14 +75,13 @@ __shared__ unsigned long long s_phase[PHASE_SLOTS];
     } while (0)
 #endif
 #define PHASE(kern, slot) PHASE_SET(kern, slot, wall_clock64())
-// k_stage1's waves per SIMD (H: its FP16 form). Exact: eight, which costs 4 spilled VGPRs and
-// is still faster than the seven of the compiler's choice (64 1080p frames 982 us against
-// 1003); FP16: six, what its registers allow. The stamps cost registers; the profiling
-// build runs six of either.
+// k_stage1's waves per SIMD: eight, which costs the exact form 4 spilled VGPRs and is still
+// faster than the seven of the compiler's choice (64 1080p frames 982 us against 1003). The
+// stamps cost registers; the profiling build runs six.
 #ifdef CCNN_PHASE_STAMPS
 #define S1_WAVES __attribute__((amdgpu_waves_per_eu(6)))
 #else
-#define S1_WAVES __attribute__((amdgpu_waves_per_eu(H ? 6 : 8)))
+#define S1_WAVES __attribute__((amdgpu_waves_per_eu(8)))
 #endif
 enum { PH_CHECK = 0, PH_STAGE1 = 1 };
 
@@ -143,6 +142,7 @@ __device__ __forceinline__ h2_t pk16(float a, float b)
 }
 
 __device__ __forceinline__ h2_t as_h2(uint32_t u) { return __builtin_bit_cast(h2_t, u); }
+__device__ __forceinline__ uint32_t as_u32(h2_t h) { return __builtin_bit_cast(uint32_t, h); }
 
 __device__ __forceinline__ float dot2(h2_t a, h2_t b, float c) { return __builtin_amdgcn_fdot2(a, b, c, false); }
 
@@ -431,8 +431,11 @@ __global__ void __launch_bounds__(256) k_level(const float* __restrict__ g, int 
 // k_stage1 28.6 -> 23.5 us. Two planes of L1 sums at a time in LDS, the other two on their
 // way meanwhile, make room for eight workgroups on a CU instead of six: k_stage1 1051 -> 982
 // us for the 64 frames, 1923 -> 1714 us for a 4800x2400 frame in 91 levels, 22.9 -> 22.0 us
-// for one 1080p frame. The FP16 form keeps its weights in memory (its products take
-// an issue slot of 4 clocks whatever their operands are) and all its planes in LDS.
+// for one 1080p frame. In the FP16 form an FP16 product pair takes an issue slot of 4 clocks
+// whatever its operands are, and so did the roundings and fused multiply-adds: L1 and L2
+// sums are rounded to FP16 once, where they enter LDS, instead of in every window that
+// holds them, and the multiply-adds have literal weights (mixed batch: k_stage1 1550 ->
+// 1290 us, k_stage1_l1 864 -> 815 us).
 // ---------------------------------------------------------------------------------
 namespace s1 {
 using N = Stage1;
@@ -626,7 +629,6 @@ __global__ void __launch_bounds__(S1A_THREADS) k_stage1_l1(const float* __restri
 
     // L1: conv_4x4 chains + lrelu_bn_max for every map, then the sums feeding L2
     // (add / add2, cnnpp_cplusplus.cpp:916-950; wiring cnn_simd_cntk.cpp:705-725)
-    [[maybe_unused]] const float* b1 = W + N::oB1;
     const size_t plane = (size_t)L.s1_w * L.s1_h;
     float* out = s1buf + L.s1_off;
     // the positions responses inside the map read (vx x vy of the tile; fewer at the
@@ -657,8 +659,7 @@ __global__ void __launch_bounds__(S1A_THREADS) k_stage1_l1(const float* __restri
                 for (int c = 0; c < 4; ++c) hp[r][c] = pk16(win[r][c] - mu, win[r][c + 1] - mu);
             const uint32_t* kh = reinterpret_cast<const uint32_t*>(W + N::SIZE) + Stage1H::oL1;
             const float* ks = W + N::SIZE + Stage1H::oS1;
-#pragma unroll
-            for (int m = 0; m < N::M1; ++m) {
+            static_for<N::M1>([&](auto m) {
                 float a[4];
                 const float acc0 = mu * ks[m];
 #pragma unroll
@@ -670,10 +671,10 @@ __global__ void __launch_bounds__(S1A_THREADS) k_stage1_l1(const float* __restri
                         acc = dot2(hp[dy + r][dx], as_h2(kh[m * 8 + 2 * r]), acc);
                         acc = dot2(hp[dy + r][dx + 2], as_h2(kh[m * 8 + 2 * r + 1]), acc);
                     }
-                    a[q] = lrelu_bn_fma(acc, b1, m, N::M1);
+                    a[q] = acc;
                 }
-                pm[m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
-            }
+                pm[m] = act_pool_fma<N, N::oB1, N::M1, m>(a[0], a[1], a[2], a[3]);
+            });
         } else {
         static_for<N::M1>([&](auto m) { pm[m] = conv4_act_pool<N, N::oK1 + m * 16, N::oB1, N::M1, m>(win); });
         }
@@ -703,21 +704,16 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     // window reads of a wave are free of bank conflicts
     constexpr int P2S = (P2W + 7) / 16 * 16 + 8, P2NS = P2S * G::P2H;
     static_assert(P2S >= P2W, "rows of L2 sums");
-    // L1 sums, PL planes at a time (exact: two, FP16: all); later the L2 sums and, on the FP16
-    // path, the tail weights. With 15.4 KB instead of 26.9 KB and 64 VGPRs eight workgroups
-    // run on a CU instead of six
-    constexpr int PL = H ? N::M1 : 2, S1N = PL * P1N > N::M2 * P2NS ? PL * P1N : N::M2 * P2NS;
-    __shared__ __align__(16) float s_s1[S1N];
-    // FP16 path: the L3, hidden- and output-layer weights, which the per-response tail
-    // reads from LDS; fetched into registers now, stored over the consumed L2 maps later
-    constexpr int WT = N::SIZE - N::oK3, WPER = (WT + S1_THREADS - 1) / S1_THREADS;
+    // Exact form: the L1 sums, two planes (PL) at a time, later the L2 sums; FP16 form: the L1
+    // sums rounded to FP16, all planes, later the L2 sums in FP16, twice: as they are and one
+    // position to the left, so that the pairs of a window at an odd column are words too
+    // (CB: where the second copy starts, in halves; the 8 keep the copies' banks apart). With
+    // 15.4 KB instead of 26.9 KB and 64 VGPRs eight workgroups run on a CU instead of six
+    constexpr int PL = H ? N::M1 : 2, CB = N::M2 * P2NS + 8;
+    constexpr int L1W = H ? PL * P1N / 2 : PL * P1N, L2W = H ? (CB + N::M2 * P2NS) / 2 : N::M2 * P2NS;
+    __shared__ __align__(16) float s_s1[L1W > L2W ? L1W : L2W];
 
     const int tid = threadIdx.x;
-    [[maybe_unused]] float wt[WPER];
-    if constexpr (H) {
-#pragma unroll
-        for (int k = 0; k < WPER; ++k) wt[k] = W[N::oK3 + min(tid + k * S1_THREADS, WT - 1)];
-    }
     const int tile = xcd_tile(blockIdx.x, gridDim.x);
     PHASE_CLEAR();
     PHASE(PH_STAGE1, 0);
@@ -775,7 +771,15 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     const auto put = [&]() {
         static_for<PER>([&](auto k) {
             const int i = tid + k * S1_THREADS;
-            if (i < NQ) *reinterpret_cast<f4_t*>(s_s1 + 4 * i) = fetched[k];
+            if (i < NQ) {
+                const f4_t v = fetched[k];
+                if constexpr (H) {
+                    const uint2 h = make_uint2(as_u32(pk16(v.x, v.y)), as_u32(pk16(v.z, v.w)));
+                    *reinterpret_cast<uint2*>(s_s1 + 2 * i) = h;
+                } else {
+                    *reinterpret_cast<f4_t*>(s_s1 + 4 * i) = v;
+                }
+            }
         });
     };
     fetch(0);
@@ -786,7 +790,6 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     // L2, one pooled L2 position per thread: the eight maps (two conv_3x3 chains per L1
     // sum + lrelu_bn_max), held in registers until every thread has read the L1 sums, whose
     // place their neighbour sums then take
-    [[maybe_unused]] const float* b2 = W + N::oB2;
     constexpr int RP = (P2W * G::P2H + S1_THREADS - 1) / S1_THREADS;   // positions per thread
     float sv[RP][N::M2];
     // the maps of the sums in LDS, from sum I0 of the network on
@@ -798,26 +801,23 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
             const int qy = (int)(((float)r + 0.5f) * rqw), qx = r - qy * qw;
             static_for<PL>([&](auto local) {
                 constexpr int i = I0 + local;
-                const float* src = s_s1 + local * P1N + (2 * qy) * P1W + 2 * qx;
-                float win[4][4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) win[r][c] = src[r * P1W + c];
                 if constexpr (H) {
-                    // pairs (c, c+1) of each window row, and (c3, 0) for the last tap of the
-                    // right-hand quads; per map and row the tap pairs (k0, k1), (k2, 0)
-                    h2_t hp[4][3], hz[4];
+                    // pairs (c, c+1) of each window row: two words, and the two halves
+                    // between them; per map and row the tap pairs (k0, k1) and (k2, 0), or
+                    // (0, k2) for the last tap of the right-hand quads
+                    const uint32_t* src = reinterpret_cast<const uint32_t*>(s_s1) + local * (P1N / 2) +
+                                          (2 * qy) * (P1W / 2) + qx;
+                    h2_t hp[4][3];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) hp[r][c] = pk16(win[r][c], win[r][c + 1]);
-                        hz[r] = pk16(win[r][3], 0.f);
+                        const uint32_t a = src[r * (P1W / 2)], b = src[r * (P1W / 2) + 1];
+                        hp[r][0] = as_h2(a);
+                        hp[r][1] = as_h2(__builtin_amdgcn_alignbit(b, a, 16));
+                        hp[r][2] = as_h2(b);
                     }
                     const uint32_t* kh = reinterpret_cast<const uint32_t*>(W + N::SIZE) + Stage1H::oL2;
-#pragma unroll
-                    for (int half = 0; half < 2; ++half) {
-                        const int m = 2 * i + half;
+                    static_for<2>([&](auto half) {
+                        constexpr int m = 2 * i + half;
                         float a[4];
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
@@ -825,14 +825,21 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
                             float acc = 0.f;
 #pragma unroll
                             for (int r = 0; r < 3; ++r) {
+                                const uint32_t k2 = kh[m * 6 + 2 * r + 1];
                                 acc = dot2(hp[dy + r][dx], as_h2(kh[m * 6 + 2 * r]), acc);
-                                acc = dot2(dx ? hz[dy + r] : hp[dy + r][2], as_h2(kh[m * 6 + 2 * r + 1]), acc);
+                                acc = dot2(hp[dy + r][2], as_h2(dx ? k2 << 16 : k2), acc);
                             }
-                            a[q] = lrelu_bn_fma(acc, b2, m, N::M2);
+                            a[q] = acc;
                         }
-                        sv[k][m] = fmaxf(fmaxf(a[0], a[1]), fmaxf(a[2], a[3]));
-                    }
+                        sv[k][m] = act_pool_fma<N, N::oB2, N::M2, m>(a[0], a[1], a[2], a[3]);
+                    });
                 } else {
+                    const float* src = s_s1 + local * P1N + (2 * qy) * P1W + 2 * qx;
+                    float win[4][4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) win[r][c] = src[r * P1W + c];
                     static_for<2>([&](auto half) {
                         constexpr int m = 2 * i + half;
                         sv[k][m] = conv3_act_pool<N, N::oK2 + m * 9, N::oB2, N::M2, m>(win);
@@ -851,30 +858,29 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     }
     __syncthreads();
     PHASE(PH_STAGE1, 2);
-    // the L2 sums over the (consumed) L1 sums; on the FP16 path the tail weights after them
+    // the L2 sums over the (consumed) L1 sums
     float* s_s2 = s_s1;
+    [[maybe_unused]] _Float16* s_h2 = reinterpret_cast<_Float16*>(s_s1);
     static_for<RP>([&](auto k) {
         const int r = tid + k * S1_THREADS;
         if (r >= nq) return;
         const int qy = (int)(((float)r + 0.5f) * rqw), qx = r - qy * qw;
         const int ps = qy * P2S + qx;
         const auto& v = sv[k];
-        s_s2[ps] = v[0] + v[1];
-#pragma unroll
-        for (int m = 1; m < N::M2 - 1; ++m) s_s2[m * P2NS + ps] = v[m - 1] + v[m] + v[m + 1];
-        s_s2[(N::M2 - 1) * P2NS + ps] = v[N::M2 - 2] + v[N::M2 - 1];
+        static_for<N::M2>([&](auto m) {
+            float sum;
+            if constexpr (m == 0) sum = v[0] + v[1];
+            else if constexpr (m == N::M2 - 1) sum = v[m - 1] + v[m];
+            else sum = v[m - 1] + v[m] + v[m + 1];
+            if constexpr (H) {
+                const _Float16 h = (_Float16)sum;
+                s_h2[m * P2NS + ps] = h;
+                if (qx > 0) s_h2[CB + m * P2NS + ps - 1] = h;
+            } else {
+                s_s2[m * P2NS + ps] = sum;
+            }
+        });
     });
-    [[maybe_unused]] float* s_wt = s_s1 + N::M2 * P2NS;
-    static_assert(!H || N::M2 * P2NS + WT + Stage1H::SIZE <= S1N, "L2 sums and tail weights fit in the L1-sum space");
-    // the L3 and hidden-layer tap pairs follow the FP32 tail weights in LDS
-    [[maybe_unused]] uint32_t* s_wh = reinterpret_cast<uint32_t*>(s_wt + WT);
-    if constexpr (H) {
-#pragma unroll
-        for (int k = 0; k < WPER; ++k)
-            if (tid + k * S1_THREADS < WT) s_wt[tid + k * S1_THREADS] = wt[k];
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(W + N::SIZE) + Stage1H::oL3;
-        for (int k = tid; k < Stage1H::SIZE - Stage1H::oL3; k += S1_THREADS) s_wh[k] = src[k];
-    }
     __syncthreads();
     PHASE(PH_STAGE1, 3);
 
@@ -895,37 +901,38 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
         oy = (int)(((float)tid + 0.5f) * rvw);
         ox = tid - oy * vw;
     }
-    const float* Wt = H ? s_wt - N::oK3 : W;   // indexed with the offsets into W
-    [[maybe_unused]] const float* b3 = Wt + N::oB3;
     float a3[N::M3];
+    [[maybe_unused]] const uint32_t* window_h =
+        reinterpret_cast<const uint32_t*>(s_h2) + (ox & 1) * (CB / 2) + oy * (P2S / 2) + (ox >> 1);
     static_for<N::M2>([&](auto i) {
-        const float* src = s_s2 + i * P2NS + oy * P2S + ox;
-        float win[N::K3H][N::K3W];
-#pragma unroll
-        for (int r = 0; r < N::K3H; ++r)
-#pragma unroll
-            for (int c = 0; c < N::K3W; ++c) win[r][c] = src[r * P2S + c];
         if constexpr (H) {
-            static_assert(N::K3W == 4, "two tap pairs per L3 row");
+            static_assert(N::K3W == 4 && P2S % 2 == 0 && CB % 2 == 0, "two tap pairs per L3 row");
+            const uint32_t* src = window_h + i * P2NS / 2;
             h2_t hp[N::K3H][2];
 #pragma unroll
             for (int r = 0; r < N::K3H; ++r) {
-                hp[r][0] = pk16(win[r][0], win[r][1]);
-                hp[r][1] = pk16(win[r][2], win[r][3]);
+                hp[r][0] = as_h2(src[r * (P2S / 2)]);
+                hp[r][1] = as_h2(src[r * (P2S / 2) + 1]);
             }
-#pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                const int m = 2 * i + half;
-                const uint32_t* kh = s_wh + (Stage1H::oL3 - Stage1H::oL3) + m * 2 * N::K3H;
+            static_for<2>([&](auto half) {
+                constexpr int m = 2 * i + half;
                 float d = 0.f;
-#pragma unroll
-                for (int r = 0; r < N::K3H; ++r) {
-                    d = dot2(hp[r][0], as_h2(kh[2 * r]), d);
-                    d = dot2(hp[r][1], as_h2(kh[2 * r + 1]), d);
-                }
-                a3[m] = lrelu_bn_fma(d, b3, m, N::M3);
-            }
+                static_for<N::K3H>([&](auto r) {
+                    constexpr int k = N::oK3 + (m * N::K3H + r) * N::K3W;
+                    d = dot2(hp[r][0], as_h2(weight_half2<N, k, k + 1>), d);
+                    d = dot2(hp[r][1], as_h2(weight_half2<N, k + 2, k + 3>), d);
+                });
+                // (maps 0 and 3 have always been rounded for the hidden layer in one step, the
+                // others from their FP32 value: results stay the same bit for bit)
+                a3[m] = lrelu_bn_fma_w<N, N::oB3, N::M3, m, m == 0 || m == 3>(d);
+            });
         } else {
+            const float* src = s_s2 + i * P2NS + oy * P2S + ox;
+            float win[N::K3H][N::K3W];
+#pragma unroll
+            for (int r = 0; r < N::K3H; ++r)
+#pragma unroll
+                for (int c = 0; c < N::K3W; ++c) win[r][c] = src[r * P2S + c];
             static_for<2>([&](auto half) {
                 constexpr int m = 2 * i + half, k = N::oK3 + m * N::K3W * N::K3H;
                 float d = 0.f;
@@ -947,17 +954,14 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
         h2_t ha[N::M3 - 1];
 #pragma unroll
         for (int j = 0; j < N::M3 - 1; ++j) ha[j] = pk16(a3[j], a3[j + 1]);
-        const uint32_t* kh = s_wh + (Stage1H::oHL - Stage1H::oL3);
-#pragma unroll
-        for (int gi = 0; gi < N::HLG; ++gi)
-#pragma unroll
-            for (int tt = 0; tt < N::HLS; ++tt) {
-                const int u = N::HLS * gi + tt;
-                float c = dot2(ha[gi], as_h2(kh[2 * u]), Wt[N::oHB + u]);
-                c = dot2(ha[gi + 2], as_h2(kh[2 * u + 1]), c);
-                c = rtanh(c * Wt[N::oHT + gi]);
-                hv[u] = __builtin_fmaf(Wt[N::oHBW + tt], __builtin_fmaf(c, 0.5f, 0.5f), Wt[N::oHBB + tt]);
-            }
+        static_for<N::HL>([&](auto u) {
+            constexpr int gi = u / N::HLS, tt = u % N::HLS, k = N::oHW + u * N::HLN;
+            float c = dot2(ha[gi], as_h2(weight_half2<N, k, k + 1>), weight_v<N, N::oHB + u>);
+            c = dot2(ha[gi + 2], as_h2(weight_half2<N, k + 2, k + 3>), c);
+            c = rtanh<false, false>(c * weight_v<N, N::oHT + gi>);
+            // fma(bn_w, fma(c, 0.5, 0.5), bn_b): the halving is exact in either factor
+            hv[u] = fma_k<__builtin_bit_cast(int, 0.5f * weight_v<N, N::oHBW + tt>)>(c + 1.f, weight_v<N, N::oHBB + tt>);
+        });
     } else {
         static_for<N::HL>([&](auto u) {
             constexpr int gi = u / N::HLS, tt = u % N::HLS;
@@ -976,15 +980,15 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     for (int gi = 0; gi < N::HLG; ++gi)
 #pragma unroll
         for (int tt = 0; tt < N::HLS; ++tt) {
-            const float wv = Wt[N::oOW + tt * N::HLG + gi];
+            const float wv = W[N::oOW + tt * N::HLG + gi];
             if (gi == 0 && tt == 0) o = hv[0] * wv;
             else if (H) o = __builtin_fmaf(hv[N::HLS * gi + tt], wv, o);
             else o = hv[N::HLS * gi + tt] * wv + o;
         }
-    float c = o + Wt[N::oOB];
-    c = c * Wt[N::oOB + 1];
+    float c = o + W[N::oOB];
+    c = c * W[N::oOB + 1];
     c = rtanh(c);
-    const float af = Wt[N::oOB + 2];
+    const float af = W[N::oOB + 2];
     const float out = (af == 0.f) ? (c + 1.f) * 0.5f : af * c;
     const int e = (oy0 + oy) * L.rw + ox0 + ox;
     resp[L.resp_off + e] = out;

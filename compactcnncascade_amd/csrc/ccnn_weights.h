@@ -167,6 +167,23 @@ __device__ __forceinline__ void static_for(F&& f)
     "v_max_f32_e32 %[t0], 0, %[a0]\n v_mul_f32_e32 %[a0], %[w1], %[a0]\n"                           \
     "v_mul_f32_e32 %[t0], %[w2], %[t0]\n v_add_f32_e32 %[t0], %[bb], %[t0]\n"                       \
     "v_add_f32_e32 %[a0], %[t0], %[a0]\n"
+// the same with fused multiply-adds (the FP16 form): fma(w1, c, fma(w2, max(0, c), bn_b)).
+// v_fmamk_f32 reads two registers and a literal and issues like a multiply; v_fma_f32 with
+// three registers takes twice as long
+#define CCNN_ACT4H                                                                                  \
+    "v_add_f32_e32 %[a0], %[cb], %[a0]\n v_add_f32_e32 %[a1], %[cb], %[a1]\n"                       \
+    "v_add_f32_e32 %[a2], %[cb], %[a2]\n v_add_f32_e32 %[a3], %[cb], %[a3]\n"                       \
+    "v_mov_b32_e32 %[b], %[bb]\n"                                                                   \
+    "v_max_f32_e32 %[t0], 0, %[a0]\n v_max_f32_e32 %[t1], 0, %[a1]\n"                               \
+    "v_max_f32_e32 %[t2], 0, %[a2]\n v_max_f32_e32 %[t3], 0, %[a3]\n"                               \
+    "v_fmamk_f32 %[t0], %[t0], %[w2], %[b]\n v_fmamk_f32 %[t1], %[t1], %[w2], %[b]\n"               \
+    "v_fmamk_f32 %[t2], %[t2], %[w2], %[b]\n v_fmamk_f32 %[t3], %[t3], %[w2], %[b]\n"               \
+    "v_fmamk_f32 %[a0], %[a0], %[w1], %[t0]\n v_fmamk_f32 %[a1], %[a1], %[w1], %[t1]\n"             \
+    "v_fmamk_f32 %[a2], %[a2], %[w1], %[t2]\n v_fmamk_f32 %[a3], %[a3], %[w1], %[t3]\n"
+#define CCNN_ACT1H                                                                                  \
+    "v_add_f32_e32 %[a0], %[cb], %[a0]\n v_mov_b32_e32 %[b], %[bb]\n"                               \
+    "v_max_f32_e32 %[t0], 0, %[a0]\n v_fmamk_f32 %[t0], %[t0], %[w2], %[b]\n"                       \
+    "v_fmamk_f32 %[a0], %[a0], %[w1], %[t0]\n"
 #define CCNN_ACC                                                                                    \
     [a0] "=&v"(a0), [a1] "=&v"(a1), [a2] "=&v"(a2), [a3] "=&v"(a3), [t0] "=&v"(t0), [t1] "=&v"(t1), \
         [t2] "=&v"(t2), [t3] "=&v"(t3)
@@ -241,9 +258,34 @@ __device__ __forceinline__ float conv3_act_pool(const float (&w)[4][4])
 #undef CCNN_CONV3
 #undef CCNN_IN3
 }
+
+// The pool of lrelu_bn_fma over the four convolutions of map M, in the FP16 form. A dot
+// product's result may be read by another kind of instruction after three wait states, which
+// the compiler does not place before an assembly block: the blocks begin with four.
+#define CCNN_AFTER_DOT "s_nop 3\n"
+template <class N, int OB, int MAPS, int M>
+__device__ __forceinline__ float act_pool_fma(float a0, float a1, float a2, float a3)
+{
+    constexpr int order = act_order<N, OB, MAPS, M>();
+    float t0, t1, t2, t3, b;
+#define CCNN_ACCH                                                                                           \
+    [a0] "+v"(a0), [a1] "+v"(a1), [a2] "+v"(a2), [a3] "+v"(a3), [t0] "=&v"(t0), [t1] "=&v"(t1),             \
+        [t2] "=&v"(t2), [t3] "=&v"(t3), [b] "=&v"(b)
+    if constexpr (order > 0)
+        asm(CCNN_AFTER_DOT CCNN_MAX4 CCNN_ACT1H : CCNN_ACCH : CCNN_PAR);
+    else if constexpr (order < 0)
+        asm(CCNN_AFTER_DOT CCNN_MIN4 CCNN_ACT1H : CCNN_ACCH : CCNN_PAR);
+    else
+        asm(CCNN_AFTER_DOT CCNN_ACT4H CCNN_MAX4 : CCNN_ACCH : CCNN_PAR);
+    return a0;
+#undef CCNN_ACCH
+}
 #undef CCNN_TAP0
 #undef CCNN_TAP
 #undef CCNN_ACT4
+#undef CCNN_AFTER_DOT
+#undef CCNN_ACT4H
+#undef CCNN_ACT1H
 #undef CCNN_ACT1
 #undef CCNN_MAX4
 #undef CCNN_MIN4
@@ -251,6 +293,32 @@ __device__ __forceinline__ float conv3_act_pool(const float (&w)[4][4])
 #undef CCNN_PAR
 #undef CCNN_K
 #undef CCNN_W
+
+// x * k + y, fused, k a literal given by its bits
+template <int BITS>
+__device__ __forceinline__ float fma_k(float x, float y)
+{
+    float r;
+    asm("v_fmamk_f32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "n"(BITS), "v"(y));
+    return r;
+}
+// lrelu_bn_fma of map M; ONCE: rounded to FP16 straight from the fused sum
+template <class N, int OB, int MAPS, int M, bool ONCE>
+__device__ __forceinline__ float lrelu_bn_fma_w(float conv)
+{
+    const float c = conv + weight_v<N, OB + M>;
+    const float t = fma_k<weight_bits<N, OB + 2 * MAPS + M>>(fmaxf(0.f, c), weight_v<N, OB + 3 * MAPS + M>);
+    if constexpr (ONCE) {
+        _Float16 h;
+        asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(h) : "v"(c), "v"(weight_v<N, OB + MAPS + M>), "v"(t));
+        return (float)h;
+    }
+    return fma_k<weight_bits<N, OB + MAPS + M>>(c, t);
+}
+// two weights rounded to FP16 in one word, as Stage1H's tap pairs
+template <class N, int A, int B>
+constexpr uint32_t weight_half2 = (uint32_t)__builtin_bit_cast(unsigned short, (_Float16)ConstNetOf<N>::net.w[A]) |
+                                  (uint32_t)__builtin_bit_cast(unsigned short, (_Float16)ConstNetOf<N>::net.w[B]) << 16;
 
 // Activation and batch norm of map M of the layer whose parameters start at OB (MAPS maps),
 // as lrelu_bn: constants that are used once, which the compiler makes literals by itself.

@@ -88,3 +88,32 @@ def test_level_windows_in_every_tile_shape(api, oracle, shape):
         for (_, lw, lh, rw, rh, mode), got in zip(levels, d.last_responses()):
             level = g if mode == 2 else oracle.resize(g, int(lw), int(lh), int(mode))
             assert np.array_equal(bits(got), bits(oracle.forward(0, level))), (w, h, lw, lh, mode)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("size", SIZES)
+def test_fp16_stage1_at_tile_edges(api, oracle, size):
+    # the FP16 form against the exact one: 0.02, the bound that the FP16 form is held to
+    # against FP64 elsewhere
+    w, h = size
+    rng = np.random.default_rng(w + 7 * h)
+    smooth = np.clip(120 + 3 * np.cumsum(rng.standard_normal((h, w)), 1), 0, 255).astype(np.float32)
+    for level in ((rng.random((h, w)) * 255).astype(np.float32), smooth):
+        print("fp16 stage1", size, flush=True)
+        assert np.abs(api.stage1(level, api.FP16_BF16) - oracle.forward(0, level)).max() < 0.02
+
+
+@pytest.mark.gpu
+def test_fp16_responses_do_not_depend_on_the_tile_shape(api):
+    frame = np.random.default_rng(11).integers(0, 256, (301, 517, 3), np.uint8)
+    want = None
+    for shape in range(12):
+        d = api.FaceDetector()
+        assert d.Init(api.Param(max_image_size=(517, 301), min_face_height=30)) == 0
+        d.set_compute_precision(api.FP16_BF16)
+        d.set_tile_shape(shape)
+        print("fp16 shape", shape, flush=True)
+        d.Detect(frame)
+        got = [bits(m) for m in d.last_responses()]
+        want = want or got
+        assert len(got) == len(want) and all(np.array_equal(a, b) for a, b in zip(got, want)), shape
