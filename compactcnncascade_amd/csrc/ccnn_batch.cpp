@@ -347,12 +347,20 @@ int Detector::run_batch(const std::vector<BatchFrame>& seg, bool device_ptr, std
         B.h_ftab[fi] = F;
     }
     HIP_OK(hipMemcpyAsync(B.d_ftab, B.h_ftab, sizeof(FrameDesc) * nf, hipMemcpyHostToDevice, B.st));
-    if (!device_ptr)
+    if (!device_ptr) {
+        bool ring = false;
         for (int fi = 0; fi < nf; ++fi) {
             const BatchFrame& f = seg[fi];
             const size_t bytes = f.step * (size_t)(f.h - 1) + (size_t)f.w * f.ch;
-            HIP_OK(hipMemcpyAsync(B.d_frames + foff[fi], f.data, bytes, hipMemcpyHostToDevice, B.st));
+            if (upload_.takes(f.data, frames_n)) {
+                if (upload_.put(B.d_frames + foff[fi], f.data, bytes, B.st) < 0) return -1;
+                ring = true;
+            } else {
+                HIP_OK(hipMemcpyAsync(B.d_frames + foff[fi], f.data, bytes, hipMemcpyHostToDevice, B.st));
+            }
         }
+        if (ring && upload_.flush(B.st) < 0) return -1;
+    }
 
     // the launch sequence of the batch; ev (optional): events recorded after each group of
     // kernels (gray, proposal network, L1 sums, stage-1 tiles, compaction, checks), ev[0]

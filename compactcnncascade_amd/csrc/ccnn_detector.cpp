@@ -469,10 +469,67 @@ Detector::Detector()
     ccnn_param_default(&param);
 }
 
+bool HostUpload::takes(const uint8_t* src, size_t bytes)
+{
+    if (bytes < MIN) return false;
+    // page-locked (and any other known) memory is left to the runtime, which sends it directly
+    hipPointerAttribute_t attr;
+    if (hipPointerGetAttributes(&attr, src) != hipSuccess) (void)hipGetLastError();
+    else if (attr.type != hipMemoryTypeUnregistered) return false;
+    if (pin_) return true;
+    bool ok = halloc(pin_, dpin_, CHUNKS * CHUNK) == 0;
+    for (auto& e : ev_) ok = ok && (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess);
+    if (!ok) release();
+    return ok;
+}
+
+int HostUpload::put(uint8_t* dst, const uint8_t* src, size_t bytes, hipStream_t st)
+{
+    // chunks of equal size, so that none is a small rest
+    const size_t n = (bytes + CHUNK - 1) / CHUNK, size = n > 0 ? (bytes / n + 4095) / 4096 * 4096 : 0;
+    for (size_t o = 0; o < bytes; o += size) {
+        const size_t len = std::min(size, bytes - o);
+        const int half = at_ / HALF;
+        if (at_ % HALF == 0 && used_[half]) HIP_OK(hipEventSynchronize(ev_[half]));
+        std::memcpy(pin_ + at_ * CHUNK, src + o, len);
+        HIP_OK(launch_upload(dpin_ + at_ * CHUNK, dst + o, len, st));
+        at_ = (at_ + 1) % CHUNKS;
+        if (at_ % HALF == 0) {
+            HIP_OK(hipEventRecord(ev_[half], st));
+            used_[half] = true;
+        }
+    }
+    return 0;
+}
+
+int HostUpload::flush(hipStream_t st)
+{
+    if (at_ % HALF == 0) return 0;
+    const int half = at_ / HALF;
+    HIP_OK(hipEventRecord(ev_[half], st));
+    used_[half] = true;
+    at_ = (half + 1) % 2 * HALF;           // the next call, perhaps on another stream, begins the other half
+    return 0;
+}
+
+void HostUpload::release()
+{
+    for (int i = 0; i < 2; ++i) {
+        if (used_[i]) (void)hipEventSynchronize(ev_[i]);
+        if (ev_[i]) (void)hipEventDestroy(ev_[i]);
+        ev_[i] = nullptr;
+        used_[i] = false;
+    }
+    hfree(pin_);
+    dpin_ = nullptr;
+    at_ = 0;
+}
+
 Detector::~Detector()
 {
     release_batch();
     for (auto& s : slots_) release_slot(s);
+    upload_.release();
     for (auto& w : d_w_) dfree(w);
     for (auto& w : d_mw_) dfree(w);
     dfree(d_skip_);
@@ -855,7 +912,11 @@ int Detector::enqueue_plan(Slot& s, const ccnn_image& img, bool device_ptr, cons
     const uint8_t* src = img.data;
     if (profiling_) HIP_OK(hipEventRecord(s.ev[0], st));
     if (!device_ptr) {
-        HIP_OK(hipMemcpyAsync(s.d_img, img.data, bytes, hipMemcpyHostToDevice, st));
+        if (upload_.takes(img.data, bytes)) {
+            if (upload_.put(s.d_img, img.data, bytes, st) < 0 || upload_.flush(st) < 0) return -1;
+        } else {
+            HIP_OK(hipMemcpyAsync(s.d_img, img.data, bytes, hipMemcpyHostToDevice, st));
+        }
         src = s.d_img;
     }
     if (pre) {

@@ -72,6 +72,8 @@ hipError_t launch_net23(int stage, const float* in, int n, const float* W, float
 // The MfmaW table of a stage-2/3 network (NetShape layout w)
 void mfma_weights(const std::vector<float>& w, std::vector<float>& out);
 hipError_t launch_selftest_tanh(uint32_t lo, uint32_t hi, unsigned long long* out, hipStream_t st);
+// n bytes from page-locked host memory (as the device addresses it, 16-byte aligned) to dst
+hipError_t launch_upload(const uint8_t* pinned, uint8_t* dst, size_t n, hipStream_t st);
 hipError_t launch_export(const int* meta, const Candidate* cands, const CheckResult* results, int* hmeta,
                          Candidate* hcands, CheckResult* hresults, int cap, hipStream_t st);
 
@@ -225,6 +227,36 @@ struct BatchFrame {
     size_t step;
     bool pre;                     // gray_image_only pre-resize to gw x gh
     int gw, gh;
+};
+
+// Uploads of frames that lie in pageable host memory, from MIN bytes a call on: copied in
+// chunks into a ring of page-locked memory, from which a kernel on the caller's stream takes
+// each chunk to the device while the next is being copied. The runtime's own copy of
+// pageable memory copies and sends its chunks (1 MB, 50 us) one after the other. From MIN on:
+// eight BGRA photographs (96 MB) 5230 -> 4708 us a call, 16 frames of 1920x1080 (99 MB) 4514 ->
+// 3957 us, a 4800x2400 frame (35 MB) 5004 -> 4819 us; below it the runtime is faster (one
+// 1920x1080 frame, 6 MB: 305 us a call against 328). Bound by the host's copy (32 GB/s by one
+// thread; the GPU reads lines just written at 35 GB/s, so more threads gain nothing). Chunks
+// of 768 KB: 182 us for 6 MB against 205 with 384 KB and 230 with 1 MB.
+class HostUpload {
+public:
+    static constexpr size_t MIN = 8 << 20;
+    // whether a call that uploads `bytes` bytes from src goes through the ring
+    bool takes(const uint8_t* src, size_t bytes);
+    // queues a piece of the call on st; src may be changed when it returns
+    int put(uint8_t* dst, const uint8_t* src, size_t bytes, hipStream_t st);
+    // ends the call: its last chunks are marked on st
+    int flush(hipStream_t st);
+    void release();
+
+private:
+    static constexpr size_t CHUNK = 768 << 10;
+    static constexpr int CHUNKS = 8, HALF = CHUNKS / 2;
+    uint8_t* pin_ = nullptr;
+    uint8_t* dpin_ = nullptr;
+    int at_ = 0;                           // the next chunk of the ring
+    hipEvent_t ev_[2] = {};                // a half of the ring has been read
+    bool used_[2] = {};
 };
 
 // Device buffers and the captured graph of the batch path: every level of every frame of a
@@ -496,6 +528,7 @@ private:
     int frame_shape_ = 0;
     int batch_captures_ = 0;
     BatchArena batch_;
+    HostUpload upload_;
     std::unique_ptr<ReplayPool> pool_;   // host replay threads of the batch path
     int fa_blocks_ = 64;           // k_facial workgroups (76 KB LDS each); windows dealt round-robin
 };
