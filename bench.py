@@ -767,7 +767,12 @@ def main():
         for name, leg in legs:
             line[name] = leg()
             progress("leg %s done" % name)
-    if not args.no_cpu_baseline:
+    ref_lib = os.path.join(os.path.dirname(os.path.abspath(__file__)), "oracle", "_ref", "libccnn_ref_O3.so")
+    if not args.no_cpu_baseline and not os.path.exists(ref_lib):
+        # the compiled reference exists only where its sources are
+        line["cpu_baseline"] = None
+        progress("no compiled reference here: cpu baseline left out")
+    elif not args.no_cpu_baseline:
         cb = cpu_baseline(frames, dict(min_face=cfg["min_face"], max_face=cfg["max_face"],
                                        scale_factor=cfg["scale_factor"]), args.cpu_seconds)
         line["cpu_baseline"] = cb
