@@ -1450,7 +1450,8 @@ __device__ __forceinline__ void check_l1l2_mfma(const float* __restrict__ in, Ch
 // waits became 28: 2.9 -> 1.2 us an item), two hidden units share an item (1.5 -> 0.9 us) and
 // the outcome is taken from the first wave's registers. k_check on 1920x1080 frames of
 // ~570 items: 37.2 -> 35.2 us alone, 18.6 -> 16.6 us a frame in a batch of 64; on 640x480
-// 28.4 -> 24.0 us.
+// 28.4 -> 24.0 us. Then L1 and L2 got literal weights (ccnn_weights.h; L1 6.7 -> 4.6 us an
+// item, L2 2.4 -> 1.9): 36.5 -> 33.7 us alone, 17.1 -> 15.2 us a frame in the batch.
 // Returns {responses above thr, bits of the largest response (at least -10)} in the first
 // wave's threads; out (optional) gets the RN responses.
 template <class N, int RP = RP_EXACT>
