@@ -145,9 +145,12 @@ __global__ void __launch_bounds__(256) k_sn_bce(float* __restrict__ z, const uns
 }
 
 // The losses of several training steps, one workgroup each: the step's n shares added one
-// after the other in single precision, so that the loss is the float sum it has always
-// been (its rounding, about 6e-5 of the loss for 86,400 shares, included). Bound by the
-// chain of dependent adds, 2.5 ns each; the shares come through LDS, SN_LOSS at a time.
+// after the other in single precision. The loss has always been such a sum (of adds to one
+// address, in the order in which they came), whose rounding is 1e-6 of the loss with 5,000
+// shares and 7e-5 with 86,400. A sum without that rounding (6e-8) lies that far from the
+// losses which earlier versions report for the same training, so this kernel keeps the
+// running sum and gives it a fixed order. Gradients do not depend on it. Bound by the chain
+// of dependent adds, 2.5 ns each; the shares come through LDS, SN_LOSS at a time.
 constexpr int SN_LOSS = 8192;
 __global__ void __launch_bounds__(256) k_sn_loss(const float* __restrict__ part_loss, size_t n,
                                                  float* __restrict__ loss)

@@ -66,3 +66,33 @@ def test_training_matches_fp64_adam(api, n, batch):
     # far; the few weights whose gradient nearly cancels may differ by more
     assert np.abs(losses - want).max() <= 1e-4 * np.abs(want).max()
     assert np.mean(np.abs(p - w)) <= 1e-3 * lr
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 21, 1387), (2, 1, 43691), (64, 90, 160)])
+def test_the_loss_is_the_average_of_all_outputs(api, shape):
+    # one share of the sum, 8,192 of them (what the summing kernel takes at a time), one more,
+    # and 86,400. Every share is added with a rounding of at most 2^-24 of the sum; the losses
+    # and their way to a share take 14 more
+    import torch
+    from compactcnncascade_amd import skipnet
+    rng = np.random.default_rng(sum(shape))
+    x = rng.normal(0.0, 0.08, shape).astype(np.float32)
+    y = (rng.random((shape[0], skipnet.SLOTS) + shape[1:]) < 5e-4).astype(np.uint8)
+    p = skipnet.init_params(4)
+    print("loss", shape, flush=True)
+    loss, _ = skipnet.grad(api, p, x, y, 500.0)
+    # the forward pass and the cross-entropy in 64 bits, a few frames at a time
+    sizes = [(8, 1, 3, 3), (8,), (8, 8, 3, 3), (8,), (skipnet.SLOTS, 8, 3, 3), (skipnet.SLOTS,)]
+    w = torch.from_numpy(p).to(torch.float64)
+    w1, b1, w2, b2, w3, b3 = (q.reshape(s) for q, s in zip(w.split([int(np.prod(s)) for s in sizes]), sizes))
+    conv = torch.nn.functional.conv2d
+    want = 0.0
+    for k in range(0, shape[0], 8):
+        a = torch.from_numpy(x[k:k + 8]).to(torch.float64)[:, None]
+        z = conv(conv(conv(a, w1, b1, padding=1).relu(), w2, b2, padding=1).relu(), w3, b3, padding=1)
+        pos = torch.from_numpy(y[k:k + 8]) != 0
+        sp = z.clamp(min=0) + torch.log1p(torch.exp(-z.abs()))
+        want += float(torch.where(pos, 500.0 * (sp - z), sp).sum())
+    want /= y.size
+    shares = (y.size + 255) // 256
+    assert abs(loss - want) <= (shares + 14) * 2.0 ** -24 * want
