@@ -657,10 +657,23 @@ extern "C" int ccnn_skipnet_train(float* params, const float* x0, const unsigned
     std::vector<int> order(n);
     for (int i = 0; i < n; ++i) order[i] = i;
     std::vector<long long> off(n);
-    // the losses of the steps since `first` are still on the device
-    std::vector<float> losses(epoch_loss ? (size_t)epochs * nb : 0);
-    int kept = 0;
-    size_t first = 0;
+    // the losses of the last `kept` steps are still on the device; the epochs whose steps
+    // have all been read are written as the run goes on
+    int kept = 0, read = 0, done = 0;
+    double lsum = 0.0;
+    auto read_losses = [&]() {
+        float l[SnRun::KEEP];
+        if (r.losses(kept, l) < 0) return -1;
+        for (int k = 0; k < kept; ++k) {
+            lsum += l[k];
+            if (++read < nb) continue;
+            epoch_loss[done++] = (float)(lsum / nb);
+            read = 0;
+            lsum = 0.0;
+        }
+        kept = 0;
+        return 0;
+    };
     unsigned long long st = seed * 6364136223846793005ull + 1442695040888963407ull;
     auto rnd = [&]() {
         st = st * 6364136223846793005ull + 1442695040888963407ull;
@@ -674,19 +687,10 @@ extern "C" int ccnn_skipnet_train(float* params, const float* x0, const unsigned
         for (int b = 0; b < nb; ++b) {
             ++t;
             if (r.step(all_x.p, all_y.p, fo.p + (size_t)b * batch, pos_weight, kept, lr, t) < 0) return -1;
-            if (epoch_loss && ++kept == r.keep) {
-                if (r.losses(kept, losses.data() + first) < 0) return -1;
-                first += kept;
-                kept = 0;
-            }
+            if (epoch_loss && ++kept == r.keep && read_losses() < 0) return -1;
         }
     }
-    if (kept > 0 && r.losses(kept, losses.data() + first) < 0) return -1;
-    for (int e = 0; epoch_loss && e < epochs; ++e) {
-        double lsum = 0.0;
-        for (int b = 0; b < nb; ++b) lsum += losses[(size_t)e * nb + b];
-        epoch_loss[e] = (float)(lsum / nb);
-    }
+    if (kept > 0 && read_losses() < 0) return -1;
     SN_OK(hipDeviceSynchronize());
     SN_OK(hipMemcpy(params, r.par, sizeof(float) * NPAR, hipMemcpyDeviceToHost));
     return 0;
