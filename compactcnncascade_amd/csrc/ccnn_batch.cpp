@@ -348,11 +348,15 @@ int Detector::run_batch(const std::vector<BatchFrame>& seg, bool device_ptr, std
     }
     HIP_OK(hipMemcpyAsync(B.d_ftab, B.h_ftab, sizeof(FrameDesc) * nf, hipMemcpyHostToDevice, B.st));
     if (!device_ptr) {
+        const auto frame_bytes = [](const BatchFrame& f) { return f.step * (size_t)(f.h - 1) + (size_t)f.w * f.ch; };
+        size_t least = frames_n;
+        for (const BatchFrame& f : seg) least = std::min(least, frame_bytes(f));
         bool ring = false;
+        upload_.begin(frames_n);
         for (int fi = 0; fi < nf; ++fi) {
             const BatchFrame& f = seg[fi];
-            const size_t bytes = f.step * (size_t)(f.h - 1) + (size_t)f.w * f.ch;
-            if (upload_.takes(f.data, frames_n)) {
+            const size_t bytes = frame_bytes(f);
+            if (upload_.takes(f.data, bytes, least, frames_n)) {
                 if (upload_.put(B.d_frames + foff[fi], f.data, bytes, B.st) < 0) return -1;
                 ring = true;
             } else {

@@ -469,9 +469,9 @@ Detector::Detector()
     ccnn_param_default(&param);
 }
 
-bool HostUpload::takes(const uint8_t* src, size_t bytes)
+bool HostUpload::takes(const uint8_t* src, size_t piece, size_t least, size_t call)
 {
-    if (bytes < MIN) return false;
+    if (!worth(piece, least, call)) return false;
     // page-locked (and any other known) memory is left to the runtime, which sends it directly
     hipPointerAttribute_t attr;
     if (hipPointerGetAttributes(&attr, src) != hipSuccess) (void)hipGetLastError();
@@ -483,27 +483,32 @@ bool HostUpload::takes(const uint8_t* src, size_t bytes)
     return ok;
 }
 
-int HostUpload::put(uint8_t* dst, const uint8_t* src, size_t bytes, hipStream_t st)
+int HostUpload::send(uint8_t* dst, size_t bytes, hipStream_t st)
 {
-    // chunks of equal size, so that none is a small rest
-    const size_t n = (bytes + CHUNK - 1) / CHUNK, size = n > 0 ? (bytes / n + 4095) / 4096 * 4096 : 0;
-    for (size_t o = 0; o < bytes; o += size) {
-        const size_t len = std::min(size, bytes - o);
-        const int half = at_ / HALF;
-        if (at_ % HALF == 0 && used_[half]) HIP_OK(hipEventSynchronize(ev_[half]));
-        std::memcpy(pin_ + at_ * CHUNK, src + o, len);
-        HIP_OK(launch_upload(dpin_ + at_ * CHUNK, dst + o, len, st));
-        at_ = (at_ + 1) % CHUNKS;
-        if (at_ % HALF == 0) {
-            HIP_OK(hipEventRecord(ev_[half], st));
-            used_[half] = true;
-        }
+    HIP_OK(launch_upload(dpin_ + at_ * CHUNK, dst, bytes, st));
+    const int half = at_ / HALF;
+    at_ = (at_ + 1) % CHUNKS;
+    if (at_ % HALF == 0) {
+        HIP_OK(hipEventRecord(ev_[half], st));
+        used_[half] = true;
     }
     return 0;
 }
 
+int HostUpload::put(uint8_t* dst, const uint8_t* src, size_t bytes, hipStream_t st)
+{
+    const auto copy = [&](size_t o, const uint8_t* p, size_t n) {
+        const int half = at_ / HALF;
+        if (o == 0 && at_ % HALF == 0 && used_[half]) HIP_OK(hipEventSynchronize(ev_[half]));
+        std::memcpy(pin_ + at_ * CHUNK + o, p, n);
+        return 0;
+    };
+    return chunks_.put(dst, src, bytes, copy, [&](uint8_t* d, size_t n) { return send(d, n, st); });
+}
+
 int HostUpload::flush(hipStream_t st)
 {
+    if (chunks_.end([&](uint8_t* d, size_t n) { return send(d, n, st); }) < 0) return -1;
     if (at_ % HALF == 0) return 0;
     const int half = at_ / HALF;
     HIP_OK(hipEventRecord(ev_[half], st));
@@ -912,7 +917,8 @@ int Detector::enqueue_plan(Slot& s, const ccnn_image& img, bool device_ptr, cons
     const uint8_t* src = img.data;
     if (profiling_) HIP_OK(hipEventRecord(s.ev[0], st));
     if (!device_ptr) {
-        if (upload_.takes(img.data, bytes)) {
+        if (upload_.takes(img.data, bytes, bytes, bytes)) {
+            upload_.begin(bytes);
             if (upload_.put(s.d_img, img.data, bytes, st) < 0 || upload_.flush(st) < 0) return -1;
         } else {
             HIP_OK(hipMemcpyAsync(s.d_img, img.data, bytes, hipMemcpyHostToDevice, st));

@@ -17,6 +17,7 @@
 
 #include "ccnn.h"
 #include "ccnn_internal.h"
+#include "ccnn_upload.h"
 
 namespace ccnn {
 
@@ -229,29 +230,52 @@ struct BatchFrame {
     int gw, gh;
 };
 
-// Uploads of frames that lie in pageable host memory, from MIN bytes a call on: copied in
-// chunks into a ring of page-locked memory, from which a kernel on the caller's stream takes
-// each chunk to the device while the next is being copied. The runtime's own copy of
-// pageable memory copies and sends its chunks (1 MB, 50 us) one after the other. From MIN on:
-// eight BGRA photographs (96 MB) 5230 -> 4708 us a call, 16 frames of 1920x1080 (99 MB) 4514 ->
-// 3957 us, a 4800x2400 frame (35 MB) 5004 -> 4819 us; below it the runtime is faster (one
-// 1920x1080 frame, 6 MB: 305 us a call against 328). Bound by the host's copy (32 GB/s by one
-// thread; the GPU reads lines just written at 35 GB/s, so more threads gain nothing). Chunks
-// of 768 KB: 182 us for 6 MB against 205 with 384 KB and 230 with 1 MB.
+// Uploads of frames that lie in pageable host memory: copied in chunks into a ring of
+// page-locked memory, from which a kernel on the caller's stream takes each chunk to the
+// device while the next is being copied; frames that lie back to back on the device share
+// chunks. The runtime's own copy of pageable memory costs about 13 us a copy, and beyond 1 MB
+// it copies and sends its chunks (1 MB, 50 us) one after the other. Bound by the host's copy
+// (32 GB/s by one thread; the GPU reads lines just written at 35 GB/s, so more threads gain
+// nothing). Chunks of 768 KB: 182 us for 6 MB against 205 with 384 KB and 230 with 1 MB.
+//
+// Which uploads (microseconds a call, runtime -> ring, host frames not seen before):
+//   frames above 1 MB: 11 of 1029 KB 694 -> 600, 4 of 1280x720 (10.5 MB) 640 -> 554, 8 of
+//   1920x1080 2130 -> 1784, one 1920x1500 (8.2 MB) 435 -> 404, one 4800x2400 1455 -> 1304;
+//   frames up to 768 KB: 1200 of 64x56 (12 MB) 7000 -> 3850, 300 of 101x99 4050 -> 1280, 128 of
+//   320x240 2260 -> 1500, 24 of 499 KB 750 -> 686, 42 of 679 KB 1268 -> 1275. A chunk and a
+//   launch for each frame made the 64x56 ones slower than the runtime, 8650;
+//   frames between the two, which the runtime sends in one piece: 32 of 640x480 (28 MB) 1140
+//   -> 1183, 68 of 899 KB 2478 -> 2714; left to the runtime, unless smaller ones lie between
+//   them (24 of 640x480 and 24 of 320x240 in turn: all in the ring 1170, without the large
+//   ones 1302, by the runtime 1272);
+//   calls below 8 MB: within 8% either way (one 1920x1080 frame 346 -> 333 us on one host, 305
+//   -> 328 on another); left to the runtime.
 class HostUpload {
 public:
     static constexpr size_t MIN = 8 << 20;
-    // whether a call that uploads `bytes` bytes from src goes through the ring
-    bool takes(const uint8_t* src, size_t bytes);
-    // queues a piece of the call on st; src may be changed when it returns
+    // whether a frame of `piece` bytes does better in the ring, in a call that uploads `call`
+    // bytes whose smallest frame has `least`
+    static constexpr bool worth(size_t piece, size_t least, size_t call)
+    {
+        return call >= MIN && (piece > RUNTIME_PIECE || least <= CHUNK);
+    }
+    // whether it goes through it: worth it, from pageable memory, and there is a ring
+    bool takes(const uint8_t* src, size_t piece, size_t least, size_t call);
+    // a call of `bytes` bytes in all begins
+    void begin(size_t bytes) { chunks_.begin(bytes, CHUNK); }
+    // queues a piece of the call on st; src may be changed when it returns, dst (16-byte
+    // aligned) holds the piece after flush
     int put(uint8_t* dst, const uint8_t* src, size_t bytes, hipStream_t st);
-    // ends the call: its last chunks are marked on st
+    // ends the call: its last chunk is sent, its last chunks are marked on st
     int flush(hipStream_t st);
     void release();
 
 private:
-    static constexpr size_t CHUNK = 768 << 10;
+    int send(uint8_t* dst, size_t bytes, hipStream_t st);
+
+    static constexpr size_t CHUNK = 768 << 10, RUNTIME_PIECE = 1 << 20;
     static constexpr int CHUNKS = 8, HALF = CHUNKS / 2;
+    UploadChunks chunks_;
     uint8_t* pin_ = nullptr;
     uint8_t* dpin_ = nullptr;
     int at_ = 0;                           // the next chunk of the ring

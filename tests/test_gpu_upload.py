@@ -52,3 +52,28 @@ def test_batches_of_host_frames_match_device_frames():
         print("batch mode", mode, flush=True)
         assert [_key(r) for r in d.DetectBatch(images=frames)] == want
         assert [_key(r) for r in d.DetectBatch(images=frames[::-1])] == want[::-1]
+
+
+def test_batches_of_small_frames_share_chunks_and_arrive_whole():
+    # hundreds of frames a chunk, sizes that leave gaps between them, frames that fill a chunk's
+    # end, frames left to the runtime (900 KB, and page-locked ones) between those of the ring
+    from compactcnncascade_amd import api
+    import torch
+    rng = np.random.default_rng(7)
+    kinds = {"small": [(64, 56, 3, 700), (101, 99, 3, 90)], "mixed": [(64, 56, 3, 40), (320, 240, 3, 20), (640, 480, 3, 4),
+                                                                     (61, 63, 4, 40), (1280, 720, 3, 2)],
+             "large": [(640, 480, 3, 8), (1280, 720, 3, 3)]}
+    for name, parts in kinds.items():
+        d = api.FaceDetector()
+        assert d.Init(api.Param(max_image_size=(1280, 720), min_face_height=24, max_face_height=60)) == 0
+        frames = [rng.integers(0, 256, (h, w, c), np.uint8) for w, h, c, n in parts for _ in range(n)]
+        frames = [frames[i] for i in rng.permutation(len(frames))]
+        keep = [torch.from_numpy(f).clone().pin_memory() for f in frames]
+        some = [keep[i].numpy() if i % 5 == 3 else f for i, f in enumerate(frames)]
+        tensors = [torch.from_numpy(f).cuda() for f in frames]
+        ptrs = [(t.data_ptr(), t.shape[1], t.shape[0], t.shape[2], t.shape[1] * t.shape[2]) for t in tensors]
+        want = [_key(r) for r in d.DetectBatch(device_frames=ptrs)]
+        assert sum(f.nbytes for f in frames) > 8 << 20
+        for images in (frames, some, frames):
+            print("small frames", name, len(frames), flush=True)
+            assert [_key(r) for r in d.DetectBatch(images=images)] == want
