@@ -341,9 +341,7 @@ int Detector::run_batch(const std::vector<BatchFrame>& seg, bool device_ptr, std
         F.qw = (F.w + 15) / 16;
         F.quads_off = (int)q0;
         q0 += (long long)F.qw * F.h;
-        const uintptr_t al = F.ch == 4 ? 16 : 4;
-        F.aligned = (((uintptr_t)F.src % al) == 0 && (uintptr_t)F.step % al == 0 ? 1 : 0) |
-                    (((uintptr_t)F.src % 4) == 0 && (uintptr_t)F.step % 4 == 0 ? 2 : 0);
+        F.aligned = (uintptr_t)F.src % 4 == 0 && (uintptr_t)F.step % 4 == 0;
         B.h_ftab[fi] = F;
     }
     HIP_OK(hipMemcpyAsync(B.d_ftab, B.h_ftab, sizeof(FrameDesc) * nf, hipMemcpyHostToDevice, B.st));

@@ -120,7 +120,7 @@ struct FrameDesc {
     int gp;               // gray pitch (floats)
     int qw;               // groups of 16 pixels per row
     int quads_off;        // first group of the frame in the batch's group numbering
-    int aligned;          // bit 0: 4-byte (16-byte for BGRA) aligned rows; bit 1: 4-byte aligned rows
+    int aligned;          // 4-byte aligned rows
 };
 
 // Stage 1 runs in two launches. The first computes the four L1-sum maps (conv, act,

@@ -41,3 +41,33 @@ def test_gray_of_batches_at_block_edges(shift):
         want = oracle.gray(frames[k])
         assert got.shape == want.shape
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), FRAMES[k]
+
+
+@pytest.mark.parametrize("ch", [1, 3, 4])
+@pytest.mark.parametrize("pad", [0, 1, 4, 16])
+def test_gray_of_thumbnails(ch, pad):
+    # frames of fewer than a block's groups, several in every block: whole groups, groups that
+    # end at each pixel of a row, rows of every alignment
+    from compactcnncascade_amd import api
+    from oracle.bind import Oracle
+    import torch
+    oracle = Oracle()
+    rng = np.random.default_rng(10 * ch + pad)
+    frames, ptrs, keep = [], [], []
+    for w in list(range(48, 68)) + [80, 96]:
+        h = 51 + w % 5
+        step = w * ch + pad
+        buf = rng.integers(0, 256, (h, step), np.uint8)
+        keep.append(torch.from_numpy(buf).cuda())
+        rows = np.ascontiguousarray(buf[:, :w * ch])
+        frames.append(rows.reshape(h, w) if ch == 1 else rows.reshape(h, w, ch))
+        ptrs.append((keep[-1].data_ptr(), w, h, ch, step))
+    d = api.FaceDetector()
+    assert d.Init(api.Param(max_image_size=(128, 64), min_face_height=27, max_face_height=40)) == 0
+    n = len(frames)
+    print("thumbnails", ch, pad, flush=True)
+    for k in range(n):
+        d.DetectBatch(device_frames=[ptrs[(k + 1 + j) % n] for j in range(n)])
+        got, want = d.getGrayImage32F(api.PIPELINE_CPU), oracle.gray(frames[k])
+        assert got.shape == want.shape
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), frames[k].shape
