@@ -478,7 +478,7 @@ def phase_pass(kind, workload="fhd_min40_max240"):
         a = api.phase_stamps(1, 65536).astype(np.int64)
         a = a[(a[:, 0] > 0) & (a[:, 4] > 0)]
         t = a[:, :5] - a[:, 0].min()
-        names = ["tile lookup + L1-sum window to LDS", "L2", "L2 sums + tail weights to LDS",
+        names = ["tile lookup + L1-sum window to LDS", "L2", "L2 sums to LDS",
                  "L3 + hidden + output (thread 0)"]
         cus = len(np.unique(a[:, 20]))
         life = us(t[:, 4] - t[:, 0])

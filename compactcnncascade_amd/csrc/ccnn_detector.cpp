@@ -89,17 +89,6 @@ void append_stage1_half(std::vector<float>& w)
             h[Stage1H::oL2 + m * 6 + 2 * r] = pack_half2(k[0], k[1]);
             h[Stage1H::oL2 + m * 6 + 2 * r + 1] = pack_half2(k[2], 0.f);
         }
-    for (int m = 0; m < N::M3; ++m)
-        for (int r = 0; r < N::K3H; ++r) {
-            const float* k = &w[N::oK3 + (m * N::K3H + r) * N::K3W];
-            h[Stage1H::oL3 + (m * N::K3H + r) * 2] = pack_half2(k[0], k[1]);
-            h[Stage1H::oL3 + (m * N::K3H + r) * 2 + 1] = pack_half2(k[2], k[3]);
-        }
-    for (int u = 0; u < N::HL; ++u) {
-        const float* k = &w[N::oHW + u * N::HLN];
-        h[Stage1H::oHL + 2 * u] = pack_half2(k[0], k[1]);
-        h[Stage1H::oHL + 2 * u + 1] = pack_half2(k[2], k[3]);
-    }
     const size_t base = w.size();
     w.resize(base + Stage1H::SIZE);
     std::memcpy(&w[base], h.data(), sizeof(uint32_t) * h.size());

@@ -41,7 +41,7 @@ namespace ccnn {
 // 2 stage-2 input written, 3-8 after each barrier of the stage-2 network (L1, L2, sums,
 // L3, hidden layer, output layer), 9-14 the same for stage 3, 15 item end, 16 stage-3
 // input written; 20 hardware id, 21 item, 22 stage 3 ran. k_stage1 (per tile): 0 start,
-// 1 L1-sum window in LDS, 2 L2 done, 3 L2 sums and tail weights in LDS, 4 response
+// 1 L1-sum window in LDS, 2 L2 done, 3 L2 sums in LDS, 4 response
 // written (thread 0's), 20 hardware id.
 // The stamps collect in LDS (so that no global address stays live in registers) and go
 // to memory once, at the end of the workgroup's work (PHASE_FLUSH).
@@ -1787,6 +1787,8 @@ __device__ __forceinline__ void prepare_crop(const float* __restrict__ g, int gp
     const uint32_t sclx = ((uint32_t)cr.rcols << 12) / CW + 1;
     const uint32_t scly = ((uint32_t)cr.rrows << 12) / CH + 1;
     static_assert(CHECK_THREADS >= 256 && CHECK_THREADS % 64 == 0, "one histogram bin per thread");
+    // both tables whole: L2's weights and activation parameters, which the exact form has as
+    // literals, are 156 floats of 2252 and 2080, at most one load of a thread's nine
     WeightRegs<Stage2::SIZE> r2;
     WeightRegs<Stage3::SIZE> r3;
     if (stage) {

@@ -19,11 +19,13 @@ namespace ccnn {
 namespace {
 
 // Layout of the scratch array (floats): the level descriptor, then the stage-1 weights,
-// then the L1-sum planes.
+// then the L1-sum planes. The weights' part has a fixed size, so that the levels that fit are
+// the same whatever the weights take.
 constexpr size_t NA_DESC = 64;                                    // 256 bytes >= sizeof(LevelDesc)
-constexpr size_t NA_W = (Stage1::SIZE + Stage1H::SIZE + 63) / 64 * 64;
+constexpr size_t NA_W = 1280;
 constexpr size_t NA_PLANES = (size_t)CCNN_NOALLOC_SCRATCH_FLOATS - NA_DESC - NA_W;
 static_assert(sizeof(LevelDesc) <= NA_DESC * sizeof(float), "descriptor slot");
+static_assert(Stage1::SIZE + Stage1H::SIZE <= NA_W, "weights' part");
 
 __device__ __align__(256) float scratch[CCNN_NOALLOC_SCRATCH_FLOATS];
 
