@@ -966,9 +966,7 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
                     d = dot2(hp[r][0], as_h2(weight_half2<N, k, k + 1>), d);
                     d = dot2(hp[r][1], as_h2(weight_half2<N, k + 2, k + 3>), d);
                 });
-                // (maps 0 and 3 have always been rounded for the hidden layer in one step, the
-                // others from their FP32 value: results stay the same bit for bit)
-                a3[m] = lrelu_bn_fma_w<N, N::oB3, N::M3, m, m == 0 || m == 3>(d);
+                a3[m] = lrelu_bn_fma_w<N, N::oB3, N::M3, m>(d);
             });
         } else {
             const float* src = s_s2 + i * P2NS + oy * P2S + ox;

@@ -302,17 +302,12 @@ __device__ __forceinline__ float fma_k(float x, float y)
     asm("v_fmamk_f32 %0, %1, %2, %3" : "=v"(r) : "v"(x), "n"(BITS), "v"(y));
     return r;
 }
-// lrelu_bn_fma of map M; ONCE: rounded to FP16 straight from the fused sum
-template <class N, int OB, int MAPS, int M, bool ONCE>
+// lrelu_bn_fma of map M
+template <class N, int OB, int MAPS, int M>
 __device__ __forceinline__ float lrelu_bn_fma_w(float conv)
 {
     const float c = conv + weight_v<N, OB + M>;
     const float t = fma_k<weight_bits<N, OB + 2 * MAPS + M>>(fmaxf(0.f, c), weight_v<N, OB + 3 * MAPS + M>);
-    if constexpr (ONCE) {
-        _Float16 h;
-        asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "=v"(h) : "v"(c), "v"(weight_v<N, OB + MAPS + M>), "v"(t));
-        return (float)h;
-    }
     return fma_k<weight_bits<N, OB + MAPS + M>>(c, t);
 }
 // two weights rounded to FP16 in one word, as Stage1H's tap pairs
