@@ -283,6 +283,7 @@ __device__ __forceinline__ void gray_group(const uint8_t* __restrict__ s, int x,
 #pragma unroll
         for (int k = 0; k < 4; ++k) gray_store<CH>(g.q[k], d + 4 * k);
     } else {
+#pragma unroll 1
         for (; x + 4 <= w; x += 4, d += 4) gray_store<CH>(*reinterpret_cast<const QuadWords<CH>*>(s + (size_t)x * CH), d);
         if (x < w) gray_quad(s, x, w, CH, false, d);
     }
@@ -363,6 +364,7 @@ __global__ void __launch_bounds__(256) k_gray_batch(const FrameDesc* __restrict_
         else gray_group<1>(s, x, F.w, d);
         return;
     }
+#pragma unroll 1
     for (int k = 0; k < 4; ++k)
         if (x + 4 * k < F.w) gray_quad(s, x + 4 * k, F.w, F.ch, false, d + 4 * k);
 }
