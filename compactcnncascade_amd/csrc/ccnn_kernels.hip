@@ -75,7 +75,7 @@ __shared__ unsigned long long s_phase[PHASE_SLOTS];
     } while (0)
 #endif
 #define PHASE(kern, slot) PHASE_SET(kern, slot, wall_clock64())
-// k_stage1's waves per SIMD: eight, which costs the exact form 4 spilled VGPRs and is still
+// k_stage1's waves per SIMD: eight, which costs the exact form 3 spilled VGPRs and is still
 // faster than the seven of the compiler's choice (64 1080p frames 982 us against 1003). The
 // stamps cost registers; the profiling build runs six.
 #ifdef CCNN_PHASE_STAMPS
@@ -474,14 +474,15 @@ __global__ void __launch_bounds__(256) k_level(const float* __restrict__ g, int 
 // (ccnn_weights.h): as SGPR operands the L1 and L2 products held the stream to 0.32
 // instructions a clock of 0.44, and the tail's weights took LDS reads and 93 VGPRs. 64
 // frames of 1920x1080: k_stage1_l1 923 -> 836 us, k_stage1 1227 -> 1078 us; one frame:
-// k_stage1 28.6 -> 23.5 us. Two planes of L1 sums at a time in LDS, the other two on their
-// way meanwhile, make room for eight workgroups on a CU instead of six: k_stage1 1051 -> 982
-// us for the 64 frames, 1923 -> 1714 us for a 4800x2400 frame in 91 levels, 22.9 -> 22.0 us
-// for one 1080p frame. In the FP16 form an FP16 product pair takes an issue slot of 4 clocks
-// whatever its operands are, and so did the roundings and fused multiply-adds: L1 and L2
-// sums are rounded to FP16 once, where they enter LDS, instead of in every window that
-// holds them, and the multiply-adds have literal weights (mixed batch: k_stage1 1550 ->
-// 1290 us, k_stage1_l1 864 -> 815 us).
+// k_stage1 28.6 -> 23.5 us. Two planes of L1 sums at a time in LDS make room for eight
+// workgroups on a CU instead of six, which cover each other's loads (those of the other two
+// planes begin after the first two's products): k_stage1 1051 -> 982 us for the 64 frames,
+// 1923 -> 1714 us for a 4800x2400 frame in 91 levels, 22.9 -> 22.0 us for one 1080p frame. In
+// the FP16 form an FP16 product pair takes an issue slot of 4 clocks whatever its operands
+// are, and so did the roundings and fused multiply-adds: L1 and L2 sums are rounded to FP16
+// once, where they enter LDS, instead of in every window that holds them, and the
+// multiply-adds have literal weights (mixed batch: k_stage1 1550 -> 1290 us, k_stage1_l1 864 ->
+// 815 us).
 // ---------------------------------------------------------------------------------
 namespace s1 {
 using N = Stage1;
@@ -798,7 +799,7 @@ __global__ void __launch_bounds__(S1_THREADS) S1_WAVES k_stage1(const LevelDesc*
     // (inside the planes: s1_w = 2*TX*tiles_x + 8, s1_h = 2*TY*tiles_y + 10). Every
     // plane row and level offset is a multiple of 8 floats and 2*ox0 of 32, so the rows
     // are copied as float4; the PL planes stack as PL*P1H rows of the tile window. On the
-    // exact path the second half of the planes is on its way while the first is in use.
+    // exact path the second half of the planes follows when the first is done with.
     static_assert(P1W % 4 == 0 && (2 * TX) % 4 == 0, "float4 rows");
     constexpr int RQ = P1W / 4, NQ = PL * P1H * RQ;
     constexpr int PER = (NQ + S1_THREADS - 1) / S1_THREADS;
